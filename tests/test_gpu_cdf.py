@@ -80,6 +80,43 @@ def test_device_cdf_equals_host_cdf_on_crafted_rows(backend, case):
     assert got[0, 0] == 0 and got[0, -1] == (1 << 24)
 
 
+def tie_rows():
+    """Rows whose second sum is full of halves of its grid: f32 probabilities around 2^-29 of
+    the sum and below.  One dominant symbol at the front, in the middle or at the end, the
+    rest uniform over a band of logits, constant (the same bits again and again), or normal
+    with the spread a trained model's logits have; row lengths around the waves', windows'
+    and heads' edges."""
+    rng = np.random.default_rng(11)
+    rows = []
+    for n in (258, 320, 4096, 4097, 8200, 50280):
+        for lo, hi in ((-21.0, -19.5), (-24.0, -20.0), (-38.0, -18.0)):
+            for at in (0, n // 2, n - 1):
+                t = rng.uniform(lo, hi, n).astype(np.float32)
+                t[at] = 0.0
+                rows.append((f"band{lo:g}-at{at}", t))
+        for v in (-20.11, -20.8, -21.5, -25.0):
+            t = np.full(n, v, np.float32)
+            t[1] = 0.0
+            rows.append((f"constant{v:g}", t))
+        for sd in (2.0, 3.0, 4.0, 6.0):
+            rows.append((f"normal{sd:g}", (rng.standard_normal(n) * sd).astype(np.float32)))
+    return rows
+
+
+def test_device_cdf_equals_host_cdf_on_rows_of_ties(backend):
+    for name, row in tie_rows():
+        n = row.size
+        d_l, d_c = hip.DeviceBuffer.from_array(row), hip.DeviceBuffer((n + 1) * 4)
+        try:
+            assert backend.cdf_from_logits_device(d_l.ptr, 1, n, d_c.ptr) == ffi.BackendResult.OK
+            hip.stream_sync(backend.stream())
+            got = d_c.download(np.uint32, n + 1)
+        finally:
+            d_l.close()
+            d_c.close()
+        assert np.array_equal(got, codec.cdf_from_logits(row)), (name, n)
+
+
 def test_device_cdf_rejects_bad_sizes(backend):
     assert backend.cdf_from_logits_device(0, 1, 0, 0) == ffi.BackendResult.INVALID_ARGUMENT
     assert backend.cdf_from_logits_device(0, 1, 1 << 24, 0) == ffi.BackendResult.INVALID_ARGUMENT
