@@ -9,9 +9,8 @@
 // twins (gemv_fma.rs:98-134): eight accumulators by column residue from +0 over the
 // 8-aligned body in column order, the horizontal sum ((l0+l4)+(l2+l6)) + ((l1+l5)+(l3+l7))
 // (the tail is empty: every matrix here has whole 32-column blocks); Q8 rows fold
-// dot_g * scale_g over the column groups from +0.  Eight lanes compute one output, lane l
-// holding the reference's accumulator l, so nothing depends on the launch shape, the batch
-// or the slot.  The norms are the reference's sequential sums (rms_norm_into,
+// dot_g * scale_g over the column groups from +0.  Eight lanes of a wave hold an output's
+// eight accumulators, so nothing depends on the launch shape, the batch or the slot.  The norms are the reference's sequential sums (rms_norm_into,
 // layer_norm_into: src/domain/tensor.rs:900-908, 1390-1398), the scan takes the portable exp, and the
 // element-wise code (conv, SiLU, softplus, the d16 recurrence, the gate, softmax) is the
 // other tiers', already the CPU path's bit for bit; so the logits are the CPU path's
@@ -27,7 +26,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <type_traits>
 
 #include "mfma_common.h"
 #include "model.h"
@@ -42,14 +40,6 @@ namespace {
 
 constexpr int kEBlock = 256;      // threads (outputs) per workgroup
 constexpr int kNormMax = 1024;    // d_model limit of the loader
-
-// A RowMat stores each row in 32-column blocks interleaved by column residue: column c of
-// row r at r cols + 32 (c / 32) + 4 (c % 8) + (c % 32) / 8, so lane l of an output's eight
-// lanes finds its four columns of a block (l, l + 8, l + 16, l + 24) in one 16-byte (F32) or
-// 4-byte (Q8) run, and the eight lanes read the block's 32 columns contiguously.
-__device__ __forceinline__ size_t rowmat_index(size_t row_off, int c) {
-    return row_off + (size_t)(c & ~31) + (size_t)(4 * (c & 7) + ((c & 31) >> 3));
-}
 
 // ---------------------------------------------------------------- embedding
 
@@ -75,13 +65,13 @@ __global__ __launch_bounds__(kEBlock) void k_embed_e(EmbedEArgs a) {
     if (tok >= (uint32_t)e.rows) tok = e.rows - 1;
     const int cols = e.cols;
     float* xo = a.x + (size_t)b * cols;
-    const size_t row_off = (size_t)tok * cols;
     if (e.group == 0) {
-        for (int c = threadIdx.x; c < cols; c += kEBlock) xo[c] = ((const float*)e.w)[rowmat_index(row_off, c)];
+        for (int c = threadIdx.x; c < cols; c += kEBlock) xo[c] = ((const float*)e.w)[rowmat_at((int)tok, c, cols, false)];
     } else {
-        const float* sc = e.scales + (size_t)tok * (cols / e.group);
+        const int ng = cols / e.group;
         for (int c = threadIdx.x; c < cols; c += kEBlock)
-            xo[c] = (float)((const int8_t*)e.w)[rowmat_index(row_off, c)] * sc[c / e.group];
+            xo[c] = (float)((const int8_t*)e.w)[rowmat_at((int)tok, c, cols, true)] *
+                    e.scales[rowmat_scale_at((int)tok, c / e.group, ng)];
     }
 }
 
@@ -171,7 +161,9 @@ struct GemvEArgs {
     float* u;
     float* z;
     int di;
-    // Products 1 and 2 of a launch of three of one shape (grid z; product 0 is w, act,
+    uint32_t chunks;        // chunks of 4 C streams
+    int stride;             // LDS row stride of the staged activations
+    // Products 1 and 2 of a launch of three of one shape (grid y; product 0 is w, act,
     // out): rows w_more[z - 1], input rows act_more[z - 1], outputs from out + out_more[z - 1].
     RowMat w_more[2];
     const float* act_more[2];
@@ -184,205 +176,335 @@ __device__ __forceinline__ float madd(float w, float x, float acc) {
     return FMA ? __builtin_fmaf(w, x, acc) : acc + w * x;
 }
 
-// Lane l's four weights of the 32-column block at column c0, as exact f32.
-template <bool Q8>
-__device__ __forceinline__ void load4(const RowMat& m, size_t row_off, int c0, int l, float (&w)[4]) {
-    const size_t at = row_off + (size_t)c0 + 4 * l;
-    if (Q8) {
-        const uint32_t q = *(const uint32_t*)((const int8_t*)m.w + at);
+// One 32-column block of one tile: for each of its four columns j of every residue, x[q][j]
+// (of four streams) times w[h][j] (of the lane's row h) added to acc[h][q] in the contract's
+// arithmetic.  v_mfma_f32_4x4x1_16b_f32 is sixteen blocks of a 4 x 1 times 1 x 4 product: each
+// of its 256 outputs is one fused multiply-add, rounded once as fmaf rounds (subnormals,
+// infinities and zeros too: checked bit for bit on 21 million random operands).  That is
+// contract 2; contract 1 takes the rounded products from it (accumulator +0; an exact product
+// of -0 comes out +0, which an accumulator that starts at +0 and so never holds -0 cannot
+// tell apart) and adds them on the vector unit, eight products issued before the first add.
+// S of the four streams are live.
+template <bool FMA, int R, int C, int S>
+__device__ __forceinline__ void rank1_block(const f32x4 (&x)[C], const float (&w)[R][4], f32x4 (&acc)[R][C]) {
+    if (FMA) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) w[j] = (float)(int8_t)(q >> (8 * j));
-    } else {
-        const float4 v = *(const float4*)((const float*)m.w + at);
-        w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int q = 0; q < C; q++)
+#pragma unroll
+                for (int h = 0; h < R; h++) acc[h][q] = __builtin_amdgcn_mfma_f32_4x4x1f32(x[q][j], w[h][j], acc[h][q], 0, 0, 0);
+        return;
+    }
+    constexpr int JB = R * C <= 2 ? 4 : 8 / (R * C);
+#pragma unroll
+    for (int j0 = 0; j0 < 4; j0 += JB) {
+        f32x4 p[JB][R][C];
+#pragma unroll
+        for (int j = 0; j < JB; j++)
+#pragma unroll
+            for (int q = 0; q < C; q++)
+#pragma unroll
+                for (int h = 0; h < R; h++)
+                    p[j][h][q] = __builtin_amdgcn_mfma_f32_4x4x1f32(x[q][j0 + j], w[h][j0 + j],
+                                                                    f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < JB; j++)
+#pragma unroll
+            for (int q = 0; q < C; q++)
+#pragma unroll
+                for (int h = 0; h < R; h++)
+#pragma unroll
+                    for (int i = 0; i < S; i++) acc[h][q][i] = acc[h][q][i] + p[j][h][q][i];
     }
 }
 
-// Eight lanes compute one output (row, S streams): lane l holds accumulator l of the
-// reference's eight, the columns c = l (mod 8) of each column group in order from +0; the
-// horizontal sum ((l0+l4)+(l2+l6)) + ((l1+l5)+(l3+l7)) is formed in lane 0 of the eight
-// by three DPP adds (hsum8_lane0); Q8 rows then take sum = sum + dot * scale from +0.
-// Workgroup (bx, by) holds rows [32 bx, 32 bx + 32) and streams [S by, S by + S), the streams' input rows
-// staged in LDS.  Every operation in the contract's arithmetic (madd).  Column counts and
-// groups are whole 32-column blocks (checked at load).
-// NB > 0: the rows have exactly NB 32-column blocks, and each lane requests its whole
-// slice of the row (NB 4-byte int8 or 16-byte F32 runs) before the first product: a
-// matrix with few rows has few lanes, so each lane keeps many loads in flight.
-template <bool Q8, bool FMA, int S, int EPI, int NB>
-__global__ __launch_bounds__(kEBlock) void k_gemv_e(GemvEArgs a) {
-    extern __shared__ __align__(16) float acts[];   // [S][cols], 32-column blocks interleaved like the rows
-    const uint32_t z = blockIdx.z;
+// Lanes 0 .. 31: a of the lane plus a of lane + 32; lanes 32 .. 63: b of lane - 32 plus b of
+// the lane.  pair16: the same within each half, 16 lanes apart; pair8: within each 16, 8 apart.
+__device__ __forceinline__ float pair32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+__device__ __forceinline__ float pair16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+constexpr int kDppRowRor8 = 0x128;   // lane i of a row of 16 reads lane i ^ 8
+__device__ __forceinline__ float pair8(float a, float b, bool upper) {
+    const float keep = upper ? b : a, give = upper ? a : b;
+    return keep + dpp_move<kDppRowRor8>(give);
+}
+
+// The weights of one 32-column block: the lane's four columns of its R rows (R = 2: the tile's
+// two, R = 1: row h), and the scale that folds the column group the block ends (GB blocks a
+// group; sc is the tile's scales at the lane's output row).
+template <bool Q8, int R>
+struct TileRaw {
+    uint32_t q[R];
+    float4 f[R];
+    float sc;
+};
+template <bool Q8, int R, int GB>
+__device__ __forceinline__ TileRaw<Q8, R> tile_load(const RowMat& m, size_t t0, int k, int h, int lane, const float* sc) {
+    TileRaw<Q8, R> r;
+    const size_t blk = t0 + k;
+    if (Q8) {
+        const uint32_t* q = (const uint32_t*)m.w + (blk * 64 + lane) * 2;
+        if (R == 2) {
+            const uint2 v = *(const uint2*)q;
+            r.q[0] = v.x, r.q[R - 1] = v.y;
+        } else {
+            r.q[0] = q[h];
+        }
+        if (GB > 0) r.sc = sc[(size_t)(k / (GB > 0 ? GB : 1)) * kRowTile];
+    } else {
+#pragma unroll
+        for (int i = 0; i < R; i++) r.f[i] = ((const float4*)m.w)[blk * 128 + 64 * (R == 2 ? i : h) + lane];
+    }
+    return r;
+}
+template <bool Q8, int R>
+__device__ __forceinline__ void tile_decode(const TileRaw<Q8, R>& r, float (&w)[R][4]) {
+#pragma unroll
+    for (int h = 0; h < R; h++) {
+        if (Q8) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[h][j] = (float)(int8_t)(r.q[h] >> (8 * j));
+        } else {
+            w[h][0] = r.f[h].x, w[h][1] = r.f[h].y, w[h][2] = r.f[h].z, w[h][3] = r.f[h].w;
+        }
+    }
+}
+
+constexpr int kEWaves = kEBlock / kWave;
+constexpr int kEAhead = 8;        // 32-column blocks of weights in flight per wave
+
+// One wave computes 8 R rows x 4 C streams.  Lane 8 l + r holds the reference's accumulators
+// l of row r of each octet, one register per stream: each step of a 32-column block adds one
+// column of every residue (rank1), so an accumulator takes the columns c = l (mod 8) of a
+// column group in order from +0.  The horizontal sum ((l0+l4)+(l2+l6)) + ((l1+l5)+(l3+l7)) is
+// pair32, pair16, pair8 (each level also folds two registers into one, so lane 16 s + i ends
+// with row i of stream s); Q8 rows then take sum = sum + dot * scale from +0, in the
+// contract's arithmetic.  Workgroup: four waves of different rows, the 4 C streams' input
+// rows staged in LDS, interleaved by residue (column 32 k + 8 j + l at 32 k + 4 l + j) so that
+// a lane reads its four columns of a block at once.  GB: 32-column blocks per scale group (0:
+// the whole row is one sum).
+//
+// Bound by vector instructions once the batch fills the chip (the head of 100 F32 streams,
+// contract 1: 91 % of the cycles issue one; two thirds of them are the adds themselves), by
+// the chain of dependent products and the load latencies below that.  The version before this
+// one (eight lanes an output on the vector unit, each product reading its activation from
+// LDS) was bound by LDS.  us a launch, before and now: F32 contract 1 at 100 streams in_proj
+// 28.5 -> 19.6, x_proj 16.6 -> 6.9, out_proj 19.6 -> 12.0, head 357 -> 187; int8 groups of 64
+// contract 2 at 32 streams 14.5 -> 8.0, 14.3 -> 5.2, 17.2 -> 7.2, 87.8 -> 51.5.
+//
+// (Two workgroups a CU at least: at most 256 registers, so the products land in vector
+// registers, not in accumulation registers that the adds would have to be copied from.)
+template <bool Q8, bool FMA, int R, int C, int S, int EPI, int GB>
+__global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
+    extern __shared__ __align__(16) float acts[];   // [4 C][stride]
+    const uint32_t z = blockIdx.y;
     const RowMat& m = z == 0 ? a.w : z == 1 ? a.w_more[0] : a.w_more[1];
     const float* const act = z == 0 ? a.act : z == 1 ? a.act_more[0] : a.act_more[1];
     float* const out = z == 0 ? a.out : a.out + (z == 1 ? a.out_more[0] : a.out_more[1]);
-    const int cols = m.cols;
-    const uint32_t b0 = blockIdx.y * S;
-    for (int s = 0; s < S; s++) {
-        const uint32_t b = min(b0 + (uint32_t)s, a.n - 1);
-        const float* src = act + (size_t)b * cols;
-        for (int c = threadIdx.x; c < cols; c += kEBlock) acts[rowmat_index((size_t)s * cols, c)] = src[c];
+    const int parts = m.tiles() * (2 / R);   // tiles (R = 2) or their halves of 8 rows
+    const XcdTile job = xcd_tile(blockIdx.x, a.chunks, (uint32_t)((parts + kEWaves - 1) / kEWaves));
+    if (!job.live) return;
+    const int lane = threadIdx.x % kWave, wave = wave_index();
+    const int cols = m.cols, nb = cols / 32;
+    const int p_raw = (int)job.unit * kEWaves + wave;
+    const int part = min(p_raw, parts - 1), t = R == 2 ? part : part / 2, half = R == 2 ? 0 : part % 2;
+    const uint32_t b0 = job.part * (4 * C);
+    const size_t w0 = (size_t)t * nb;
+    // the row of the lane's outputs; R = 1: lanes 8 .. 15 of each 16 hold copies
+    const int r16 = R == 2 ? lane % 16 : 8 * half + lane % 8;
+    const int r = t * kRowTile + r16;
+    const bool row_live = p_raw < parts && r < m.rows && (R == 2 || (lane & 8) == 0);
+    constexpr int kGB = GB > 0 ? GB : 1;   // (no division by zero in the other instantiation)
+    const int ng = GB > 0 ? nb / kGB : 1;
+    const float* scales = Q8 ? m.scales + (size_t)t * ng * kRowTile + r16 : nullptr;
+    TileRaw<Q8, R> raw[kEAhead];
+#pragma unroll
+    for (int i = 0; i < kEAhead; i++) raw[i] = tile_load<Q8, R, GB>(m, w0, min(i, nb - 1), half, lane, scales);
+    const float sc_row = Q8 && GB == 0 ? scales[0] : 0.0f;
+    // the epilogue's operands, requested with the products'
+    float old[C], cs[C][3], cb = 0.0f;
+    float4 cw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    size_t cst[C];
+    const bool conv = EPI == kEpiIn && row_live && r < a.di;
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+        const uint32_t b = b0 + 4 * q + (uint32_t)lane / 16;
+        old[q] = EPI == kEpiRes && row_live && b < a.n ? out[(size_t)b * a.ostride + r] : 0.0f;
+        cs[q][0] = cs[q][1] = cs[q][2] = 0.0f;
+        cst[q] = 0;
+        if (conv && b < a.n) {
+            cst[q] = ((size_t)clamp_slot(a.slots[b], a.scap) * a.di + r) * 3;
+#pragma unroll
+            for (int k = 0; k < 3; k++) cs[q][k] = a.conv_st[cst[q] + k];
+        }
+    }
+    if (conv) {
+        cw = *(const float4*)(a.conv_w + (size_t)r * 4);
+        cb = a.conv_b[r];
+    }
+    const int stride = a.stride;
+#pragma unroll
+    for (int s = 0; s < C; s++) {
+        const int sr = wave + kEWaves * s;   // the wave's streams; S == 1: only the first is read
+        const float* src = act + (size_t)min(b0 + (uint32_t)sr, a.n - 1) * cols;
+        if (S == 4 || sr < S) {
+#pragma unroll 3
+            for (int q = lane; q < cols / 4; q += kWave) {
+                const float* p = src + 32 * (q / 8) + q % 8;
+                const float4 v = make_float4(p[0], p[8], p[16], p[24]);
+                *(float4*)(acts + sr * stride + 4 * q) = v;
+            }
+        }
     }
     __syncthreads();
-    const int l = (int)threadIdx.x % 8;
-    const int r_raw = (int)blockIdx.x * (kEBlock / 8) + (int)threadIdx.x / 8;
-    const bool live = r_raw < m.rows;
-    const int r = live ? r_raw : m.rows - 1;   // every lane joins the horizontal sums
-    const size_t row_off = (size_t)r * cols;
-    const int group = Q8 ? m.group : cols;
-    const int ng = cols / group;
-    float res[S];
+    const float* xa = acts + (S == 1 ? 0 : lane % 4) * stride + 4 * (lane / 8);
+    f32x4 acc[R][C];
+    float res[C];
 #pragma unroll
-    for (int s = 0; s < S; s++) res[s] = 0.0f;
-    // The eight lanes' horizontal sum of each stream's accumulator, then the group's fold
-    // (both complete in lane 0 of the eight, the lane that stores).
-    auto finish_group = [&](float (&acc)[S], int g) {
+    for (int q = 0; q < C; q++) {
 #pragma unroll
-        for (int s = 0; s < S; s++) {
-            const float v = hsum8_lane0(acc[s]);
-            res[s] = Q8 ? madd<FMA>(v, m.scales[(size_t)r * ng + g], res[s]) : v;
-            acc[s] = 0.0f;
+        for (int h = 0; h < R; h++) acc[h][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        res[q] = 0.0f;
+    }
+    auto finish = [&](float sc) {
+#pragma unroll
+        for (int q = 0; q < C; q++) {
+            float h2[R];
+#pragma unroll
+            for (int h = 0; h < R; h++) {
+                const f32x4 v = acc[h][q];
+                h2[h] = S == 1 ? pair16(pair32(v[0], v[0]), pair32(v[0], v[0]))
+                               : pair16(pair32(v[0], v[2]), pair32(v[1], v[3]));
+                acc[h][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            const float v = pair8(h2[0], h2[R - 1], (lane & 8) != 0);
+            res[q] = Q8 ? madd<FMA>(v, sc, res[q]) : v;
         }
     };
-    if constexpr (NB > 0) {
-        typedef typename std::conditional<Q8, uint32_t, float4>::type Raw;
-        Raw raw[NB];
+    f32x4 x[C];
 #pragma unroll
-        for (int i = 0; i < NB; i++) {
-            const size_t at = row_off + 32 * (size_t)i + 4 * l;
-            if constexpr (Q8)
-                raw[i] = *(const uint32_t*)((const int8_t*)m.w + at);
-            else
-                raw[i] = *(const float4*)((const float*)m.w + at);
+    for (int q = 0; q < C; q++) x[q] = *(const f32x4*)(xa + (4 * q) * stride);
+    // (the next block's activations are requested before this block's products)
+    auto block = [&](const TileRaw<Q8, R>& rw, int k) {
+        f32x4 xn[C];
+#pragma unroll
+        for (int q = 0; q < C; q++) xn[q] = *(const f32x4*)(xa + (4 * q) * stride + 32 * min(k + 1, nb - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        float w[R][4];
+        tile_decode<Q8, R>(rw, w);
+        rank1_block<FMA, R, C, S>(x, w, acc);
+        if (GB > 0 && (k + 1) % kGB == 0) finish(rw.sc);
+#pragma unroll
+        for (int q = 0; q < C; q++) x[q] = xn[q];
+    };
+    const int nbm = nb / kEAhead * kEAhead;
+    for (int k0 = 0; k0 < nbm; k0 += kEAhead) {
+#pragma unroll
+        for (int i = 0; i < kEAhead; i++) {
+            block(raw[i], k0 + i);
+            raw[i] = tile_load<Q8, R, GB>(m, w0, min(k0 + kEAhead + i, nb - 1), half, lane, scales);
         }
-        const int bpg = group / 32;
-        float acc[S];
-#pragma unroll
-        for (int s = 0; s < S; s++) acc[s] = 0.0f;
-        int g = 0;
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-            float w[4];
-            if constexpr (Q8) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) w[j] = (float)(int8_t)(raw[i] >> (8 * j));
-            } else {
-                w[0] = raw[i].x, w[1] = raw[i].y, w[2] = raw[i].z, w[3] = raw[i].w;
-            }
-#pragma unroll
-            for (int s = 0; s < S; s++) {
-                const float4 x = *(const float4*)(acts + (size_t)s * cols + 32 * i + 4 * l);
-                acc[s] = madd<FMA>(w[0], x.x, acc[s]);
-                acc[s] = madd<FMA>(w[1], x.y, acc[s]);
-                acc[s] = madd<FMA>(w[2], x.z, acc[s]);
-                acc[s] = madd<FMA>(w[3], x.w, acc[s]);
-            }
-            if ((i + 1) % bpg == 0) finish_group(acc, g++);
-        }
-    } else
-    for (int g = 0; g < ng; g++) {
-        const int c0 = g * group;
-        float acc[S];
-#pragma unroll
-        for (int s = 0; s < S; s++) acc[s] = 0.0f;
-#pragma unroll 4
-        for (int c = c0; c < c0 + group; c += 32) {
-            float w[4];
-            load4<Q8>(m, row_off, c, l, w);
-#pragma unroll
-            for (int s = 0; s < S; s++) {
-                const float4 x = *(const float4*)(acts + (size_t)s * cols + c + 4 * l);
-                acc[s] = madd<FMA>(w[0], x.x, acc[s]);
-                acc[s] = madd<FMA>(w[1], x.y, acc[s]);
-                acc[s] = madd<FMA>(w[2], x.z, acc[s]);
-                acc[s] = madd<FMA>(w[3], x.w, acc[s]);
-            }
-        }
-        finish_group(acc, g);
     }
-    if (!live || l != 0) return;
+    // the last nb % kEAhead blocks, already in raw[0 ..]
 #pragma unroll
-    for (int s = 0; s < S; s++) {
-        const uint32_t b = b0 + (uint32_t)s;
-        if (b >= a.n) break;
-        const float y = res[s];
+    for (int i = 0; i < kEAhead - 1; i++)
+        if (nbm + i < nb) block(raw[i], nbm + i);
+    if (GB == 0) finish(sc_row);
+    if (!row_live) return;
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+        const uint32_t b = b0 + 4 * q + (uint32_t)lane / 16;
+        if (b >= a.n) continue;
+        const float y = res[q];
         if (EPI == kEpiPlain) {
             out[(size_t)b * a.ostride + r] = y;
         } else if (EPI == kEpiRes) {
             // x += W_out * gated (model.rs:714-719): the residual add after the projection
-            float* xp = out + (size_t)b * a.ostride + r;
-            *xp = *xp + y;
+            out[(size_t)b * a.ostride + r] = old[q] + y;
         } else if (EPI == kEpiRelu2) {
             // squared_relu_into (tensor.rs:1386-1388): max(y, 0)^2, a NaN to 0
-            const float t = y > 0.0f ? y : 0.0f;
-            out[(size_t)b * a.ostride + r] = t * t;
+            const float v = y > 0.0f ? y : 0.0f;
+            out[(size_t)b * a.ostride + r] = v * v;
         } else if (r >= a.di) {
             a.z[(size_t)b * a.di + (r - a.di)] = y;
         } else {
             // conv_silu_block (model.rs:134-153) for channel r of stream b, then SiLU with the
             // lane sigmoid: d_inner comes in whole 64-channel blocks, so every channel is in
             // the 8-aligned body of its 256-channel block (tensor.rs:1197-1211).
-            const uint32_t slot = clamp_slot(a.slots[b], a.scap);
-            float* st = a.conv_st + ((size_t)slot * a.di + r) * 3;
-            const float4 cw = *(const float4*)(a.conv_w + (size_t)r * 4);
-            const float s0 = st[0], s1 = st[1], s2 = st[2];
+            float* st = a.conv_st + cst[q];
             float val = 0.0f;
-            val += s0 * cw.x;
-            val += s1 * cw.y;
-            val += s2 * cw.z;
+            val += cs[q][0] * cw.x;
+            val += cs[q][1] * cw.y;
+            val += cs[q][2] * cw.z;
             val += y * cw.w;
-            val += a.conv_b[r];
-            st[0] = s1;
-            st[1] = s2;
+            val += cb;
+            st[0] = cs[q][1];
+            st[1] = cs[q][2];
             st[2] = y;
             a.u[(size_t)b * a.di + r] = val * lane_sigmoid_f(val);
         }
     }
 }
 
-template <int S, int EPI, int NB>
-const void* gemv_e_fn(bool q8, bool fma) {
-    if (q8) return fma ? (const void*)k_gemv_e<true, true, S, EPI, NB> : (const void*)k_gemv_e<true, false, S, EPI, NB>;
-    return fma ? (const void*)k_gemv_e<false, true, S, EPI, NB> : (const void*)k_gemv_e<false, false, S, EPI, NB>;
+template <int R, int C, int S, int EPI>
+const void* gemv_e_fn(const RowMat& w, bool fma) {
+    if (w.group == 0) return fma ? (const void*)k_gemv_e<false, true, R, C, S, EPI, 0> : (const void*)k_gemv_e<false, false, R, C, S, EPI, 0>;
+    if (w.group == w.cols) return fma ? (const void*)k_gemv_e<true, true, R, C, S, EPI, 0> : (const void*)k_gemv_e<true, false, R, C, S, EPI, 0>;
+    return fma ? (const void*)k_gemv_e<true, true, R, C, S, EPI, 2> : (const void*)k_gemv_e<true, false, R, C, S, EPI, 2>;
 }
 
-// The row slice in flight whole for Mamba-130M's widths (768 and 1536 columns), the
-// generic loop for the others and for F32 batches (a whole F32 slice of 1536 columns
-// takes 200 registers: two waves per SIMD, slower from a few streams on).
-template <int S, int EPI>
-const void* gemv_e_nb(int cols, bool q8, bool fma) {
-    if (!q8 && S > 1) return gemv_e_fn<S, EPI, 0>(q8, fma);
-    if (cols == 768) return gemv_e_fn<S, EPI, 24>(q8, fma);
-    if (cols == 1536) return gemv_e_fn<S, EPI, 48>(q8, fma);
-    return gemv_e_fn<S, EPI, 0>(q8, fma);
-}
-
+// A wave's share of a product: 8 R rows and 4 C streams.
+struct Share {
+    int r, c;
+};
+typedef const void* (*GemvPick)(uint32_t n, Share s, const RowMat& w, bool fma);
 template <int EPI>
-const void* gemv_e_pick(uint32_t s, int cols, bool q8, bool fma) {
-    if (s == 8) return gemv_e_nb<8, EPI>(cols, q8, fma);
-    return s == 1 ? gemv_e_nb<1, EPI>(cols, q8, fma) : gemv_e_nb<4, EPI>(cols, q8, fma);
+const void* gemv_e_pick(uint32_t n, Share s, const RowMat& w, bool fma) {
+    if (s.r == 1) return n == 1 ? gemv_e_fn<1, 1, 1, EPI>(w, fma) : gemv_e_fn<1, 1, 4, EPI>(w, fma);
+    return s.c == 1 ? gemv_e_fn<2, 1, 4, EPI>(w, fma) : gemv_e_fn<2, 2, 4, EPI>(w, fma);
 }
 
-// Streams per workgroup: one for a single stream, four otherwise (their input rows in LDS:
-// 4 x d_inner floats at most 32 KB; sixteen, reading each row once per 16 streams, leave
-// too few workgroups: 32 streams 1.78 -> 2.38 ms per step; eight at 64 and 128 streams
-// double the out_proj time).  The head, with 50K rows, takes eight from 16 streams on
-// (its weights read half as often: Mamba-130M F32 at 128 streams 643 -> 422 us; sixteen
-// 597 us).  A stream's arithmetic does not depend on it.
-uint32_t exact_streams(uint32_t n) { return n == 1 ? 1u : 4u; }
-constexpr uint32_t kHeadStreams = 8;
+constexpr uint32_t kELdsMax = 64 * 1024;
+// LDS row stride of the staged activations: 32 words more than the row, so that the four
+// streams of a quad start in alternating halves of the banks; the row alone where that would
+// not fit (4,096 columns).
+int acts_stride(int cols, int quads) {
+    return 16 * (uint32_t)quads * (uint32_t)(cols + 32) <= kELdsMax ? cols + 32 : cols;
+}
 
-Launch gemv_e_launch(const void* (*pick)(uint32_t, int, bool, bool), bool fma, int cls, const RowMat& w,
-                     const float* act, uint32_t n, GemvEArgs a, uint32_t s_wide = 0, uint32_t products = 1) {
-    // s_wide streams per workgroup once the batch fills two such workgroups
-    const uint32_t S = s_wide && n >= 2 * s_wide ? s_wide : exact_streams(n);
-    const void* fn = pick(S, w.cols, w.group != 0, fma);
+// The smallest share (8 rows x 4 streams) up to ten waves a SIMD, since a lone wave issues at
+// a third of the vector rate and its chain of products is the kernel's time; above that 16
+// rows x 8 streams, which reads each operand half as often.  us a launch, shares of 8 x 4,
+// 8 x 8, 16 x 4, 16 x 8, 16 x 16 (Mamba-130M; F32 contract 1 at 100 streams, then int8 groups
+// of 64 contract 2 at 32): in_proj 19.6, 19.7, 19.6, 20.1, 25.3 and 8.0, 8.7, 8.1, 8.7, 13.2;
+// x_proj 6.9, 10.9, 10.0, 16.4 and 5.2, 7.0, 6.8, 8.6; out_proj 12.0, 13.8, 14.4, 17.0 and 7.2,
+// 9.4, 8.8, 12.0; the head 229, 191, 218, 187, 200 and 67.6, 55.4, 55.6, 51.5, 53.7.
+Share exact_share(const RowMat& w, uint32_t products, uint32_t n) {
+    const uint64_t waves = (uint64_t)w.tiles() * 2 * products * ((n + 3) / 4);
+    if (waves <= 10 * 1024) return Share{1, 1};
+    return Share{2, 32u * (uint32_t)w.cols <= kELdsMax ? 2 : 1};
+}
+
+Launch gemv_e_launch(GemvPick pick, bool fma, int cls, const RowMat& w, const float* act, uint32_t n, GemvEArgs a,
+                     uint32_t products = 1) {
+    const Share s = exact_share(w, products, n);
     a.w = w;
     a.act = act;
     a.n = n;
-    const uint32_t lds = S * (uint32_t)w.cols * 4u;
-    constexpr int rows_per_wg = kEBlock / 8;
-    return Launch::make(fn, dim3((unsigned)((w.rows + rows_per_wg - 1) / rows_per_wg), (n + S - 1) / S, products),
-                        dim3(kEBlock), lds, (uint32_t)cls, a);
+    a.chunks = (n + 4 * s.c - 1) / (4 * s.c);
+    a.stride = acts_stride(w.cols, s.c);
+    const uint32_t lds = 16u * (uint32_t)s.c * (uint32_t)a.stride;
+    const uint32_t units = (uint32_t)((w.tiles() * (2 / s.r) + kEWaves - 1) / kEWaves);
+    return Launch::make(pick(n, s, w, fma), dim3(xcd_grid(a.chunks, units), products), dim3(kEBlock), lds,
+                        (uint32_t)cls, a);
 }
 
 }  // namespace
@@ -392,10 +514,10 @@ Launch exact_gemv_launch(const RowMat& w, const float* act, uint32_t n, float* o
     GemvEArgs a{};
     a.out = out;
     a.ostride = ostride;
-    const void* (*pick)(uint32_t, int, bool, bool) = epi == EXACT_RESID   ? gemv_e_pick<kEpiRes>
-                                                      : epi == EXACT_RELU2 ? gemv_e_pick<kEpiRelu2>
-                                                                           : gemv_e_pick<kEpiPlain>;
-    return gemv_e_launch(pick, false, (int)cls, w, act, n, a, cls == KC_HEAD ? kHeadStreams : 0);
+    const GemvPick pick = epi == EXACT_RESID   ? gemv_e_pick<kEpiRes>
+                          : epi == EXACT_RELU2 ? gemv_e_pick<kEpiRelu2>
+                                               : gemv_e_pick<kEpiPlain>;
+    return gemv_e_launch(pick, false, (int)cls, w, act, n, a);
 }
 
 Launch exact_gemv3_launch(const RowMat* const (&w)[3], const float* const (&act)[3], uint32_t n, float* out,
@@ -408,7 +530,7 @@ Launch exact_gemv3_launch(const RowMat* const (&w)[3], const float* const (&act)
         a.act_more[k] = act[k + 1];
         a.out_more[k] = out_off[k + 1] - out_off[0];
     }
-    return gemv_e_launch(gemv_e_pick<kEpiPlain>, false, (int)cls, *w[0], act[0], n, a, 0, 3);
+    return gemv_e_launch(gemv_e_pick<kEpiPlain>, false, (int)cls, *w[0], act[0], n, a, 3);
 }
 
 void ExactStep::build(Pool& p, const StepIO& io, std::vector<Launch>& out, int& io_i, int& head_i, int& sm_i) const {
@@ -453,7 +575,7 @@ void ExactStep::build(Pool& p, const StepIO& io, std::vector<Launch>& out, int& 
     GemvEArgs gh{};
     gh.out = io.out;
     gh.ostride = D.vocab;
-    out.push_back(gemv_e_launch(gemv_e_pick<kEpiPlain>, fma, KC_HEAD, *m.head, p.normed, n, gh, kHeadStreams));
+    out.push_back(gemv_e_launch(gemv_e_pick<kEpiPlain>, fma, KC_HEAD, *m.head, p.normed, n, gh));
     sm_i = -1;
     if (io.probs) {
         sm_i = (int)out.size();

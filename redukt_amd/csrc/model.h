@@ -53,16 +53,33 @@ struct GMat {
     size_t bytes() const;
 };
 
-// A row-major [rows][cols] matrix for the reference-order tier: F32, or int8 with one f32
-// scale per `group` columns ([rows][cols / group]), the layout of the reference's own
-// Q8wMatrix (src/domain/gemv.rs:244-273).
+// A [rows][cols] matrix for the reference-order tier: F32, or int8 with one f32 scale per
+// `group` columns (the values of the reference's own Q8wMatrix, src/domain/gemv.rs:244-273),
+// in the operand order of v_mfma_f32_4x4x1_16b_f32.  Rows are padded to whole 16-row tiles
+// (zeros); columns come in whole 32-column blocks.  Lane 8 l + r of a wave owns, of tile t and
+// block k, the columns of residue l (mod 8) of rows 16 t + r and 16 t + 8 + r:
+//   Q8 : [t][k][lane][h][j] int8       — 8 bytes per lane and block
+//   F32: [t][k][h][lane][j] f32        — two 16-byte runs per lane and block
+// holding W[16 t + 8 h + r][32 k + 8 j + l], j = 0 .. 3, so every load of a wave is one
+// contiguous run.  Q8 scales: [t][cols / group][16 rows].
 struct RowMat {
     int rows = 0, cols = 0;
     int group = 0;        // 0: F32; Q8: columns per scale
     void* w = nullptr;
     float* scales = nullptr;
-    size_t bytes() const { return w ? (size_t)rows * cols * (group ? 1 : 4) + (group ? (size_t)rows * (cols / group) * 4 : 0) : 0; }
+    __host__ __device__ int tiles() const { return (rows + kRowTile - 1) / kRowTile; }
+    size_t padded() const { return (size_t)tiles() * kRowTile; }
+    size_t bytes() const { return w ? padded() * cols * (group ? 1 : 4) + (group ? padded() * (cols / group) * 4 : 0) : 0; }
 };
+// Where a RowMat keeps row r, column c, and the scale of row r, column group g (of ng).
+__host__ __device__ inline size_t rowmat_at(int r, int c, int cols, bool q8) {
+    const size_t blk = (size_t)(r / kRowTile) * (cols / 32) + c / 32;
+    const int h = r / 8 % 2, lane = 8 * (c % 8) + r % 8, j = c % 32 / 8;
+    return q8 ? (blk * 64 + lane) * 8 + 4 * h + j : ((blk * 2 + h) * 64 + lane) * 4 + j;
+}
+__host__ __device__ inline size_t rowmat_scale_at(int r, int g, int ng) {
+    return ((size_t)(r / kRowTile) * ng + g) * kRowTile + r % kRowTile;
+}
 
 struct DLayer {
     float* norm_w = nullptr;

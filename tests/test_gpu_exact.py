@@ -217,3 +217,33 @@ def test_exact_tier_refuses_what_it_does_not_serve(small):
     assert lib.lib.redukt_backend_init_ex(small["base"].encode(), 0, 256, ffi.ctypes.byref(info)) == \
         ffi.BackendResult.INVALID_ARGUMENT
     lib.lib.redukt_backend_free()
+
+
+@pytest.mark.parametrize("profile", [EXACT, ffi.PROFILE_Q8_G64 | EXACT | FMA, ffi.PROFILE_Q8_ROW | EXACT])
+def test_streams_keep_their_bits_in_every_share(tmp_path, profile):
+    """The projections take 8 rows x 4 streams a wave, or 16 x 8 where there are many rows (a
+    50,283-row head from 5 streams on, a ragged last tile): at batch sizes around the quads'
+    edges a stream's logits are those of the stream alone, which takes one stream a wave and
+    is the oracle's bit for bit."""
+    dims = rbin.MambaDims(vocab=50283, d_model=96, n_layer=1)
+    path = str(tmp_path / "wide.rbin")
+    synth.write_synthetic_mamba(path, dims, seed=21)
+    rng = np.random.default_rng(4)
+    toks = synth.zipf_tokens(rng, dims.vocab, (2, 17))
+    orc_profile = (profile & 3) | (O.ORC_PROFILE_FMA if profile & FMA else 0)
+    with ffi.PluginBackend(path, profile=profile) as be:
+        be.batch_init(17)
+        alone = np.empty((2, 17, dims.vocab), np.float32)
+        orc = O.MambaOracle(path, orc_profile, cap=17)
+        for t in range(2):
+            for s in range(17):
+                be.forward_batch([s], [int(toks[t, s])], alone[t, s])
+            c = orc.forward(list(range(17)), [int(x) for x in toks[t]])
+            assert np.array_equal(bits(alone[t]), bits(c)), t
+        orc.close()
+        for n in (2, 3, 4, 5, 8, 9, 16, 17):
+            be.batch_reset()
+            for t in range(2):
+                g = np.empty((n, dims.vocab), np.float32)
+                be.forward_batch(list(range(n)), [int(x) for x in toks[t, :n]], g)
+                assert np.array_equal(bits(g), bits(alone[t, :n])), (n, t)
