@@ -110,6 +110,9 @@ __device__ __forceinline__ float prob_of(double e, double inv_sum) { return (flo
 
 constexpr uint32_t kSpan = 16;                      // consecutive elements per thread in a chunk
 constexpr uint32_t kChunk = kSpan * kCdfBlock;      // elements per chunk workgroup
+constexpr uint32_t kTerms = 4;                      // consecutive elements per lane of a segment
+constexpr uint32_t kSegTerms = 64 * kTerms;         // elements of a segment of the sums: one wave's
+__host__ __device__ constexpr uint32_t segments(uint32_t n) { return (n + kSegTerms - 1) / kSegTerms; }
 
 struct ChunkPart {
     double max;        // the chunk's max (NaN loses; -inf if none)
@@ -124,6 +127,7 @@ struct CdfArgs {
     uint32_t rows, n, chunks;
     double* e;             // [rows][n] scratch: exp(logit - max)
     double* sums;          // [rows][2] scratch: sum of e, sum of the probabilities
+    double* seg;           // [rows][segments] scratch: sum of each kSegTerms elements of e, in any order
     ChunkPart* part;       // [rows][chunks] scratch
     uint32_t* cdf;         // [rows][n + 1]
 };
@@ -144,6 +148,28 @@ __device__ T block_reduce(T v, F op, T* sh) {
     for (int i = 1; i < kCdfBlock / 64; i++) r = op(r, sh[i]);
     __syncthreads();
     return r;
+}
+
+// A 64-bit value moved across lanes by DPP (each 32-bit half; lanes without a source
+// read 0): a few cycles, against an LDS round trip for a lane permute.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const uint64_t b = as_u64(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
+    return as_f64(((uint64_t)hi << 32) | lo);
+}
+
+// Inclusive prefix sum over the wave's 64 lanes: shifts by 1, 2, 4, 8 within each row of
+// 16 lanes, then the last lane of row 0 / 2 into rows 1 / 3 and lane 31 into rows 2 and 3.
+__device__ __forceinline__ double wave_incl_sum(double v) {
+    v += dpp_f64<0x111>(v);          // row_shr:1
+    v += dpp_f64<0x112>(v);          // row_shr:2
+    v += dpp_f64<0x114>(v);          // row_shr:4
+    v += dpp_f64<0x118>(v);          // row_shr:8
+    v += dpp_f64<0x142, 0xa>(v);     // row_bcast:15 into rows 1 and 3
+    v += dpp_f64<0x143, 0xc>(v);     // row_bcast:31 into rows 2 and 3
+    return v;
 }
 
 __device__ __forceinline__ double max_nan_loses(double m, double v) { return (!isnan(v) && !(v <= m)) ? v : m; }
@@ -177,7 +203,9 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_max(CdfArgs a) {
     if (threadIdx.x == 0) a.part[(size_t)row * a.chunks + c].max = m;
 }
 
-// Phase 1b (chunk c of row r): the row's max from the chunk maxima, then e = exp(logit - max).
+// Phase 1b (chunk c of row r): the row's max from the chunk maxima, then e = exp(logit - max),
+// and each segment's sum of e (a wave's elements of one iteration), which only guides
+// k_cdf_sums.
 __global__ __launch_bounds__(kCdfBlock) void k_cdf_exp(CdfArgs a) {
     const uint32_t c = blockIdx.x, row = blockIdx.y, n = a.n;
     const ChunkPart* pr = a.part + (size_t)row * a.chunks;
@@ -185,20 +213,31 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_exp(CdfArgs a) {
     for (uint32_t i = 1; i < a.chunks; i++) m = (pr[i].max <= m) ? m : pr[i].max;
     const float* l = a.logits + (size_t)row * n;
     double* e = a.e + (size_t)row * n;
-    const uint32_t i0 = c * kChunk, i1 = min(n, (c + 1) * kChunk);
-    if (vec_row(l) && ((uintptr_t)e & 15) == 0) {
-        for (uint32_t i = i0 + 4 * threadIdx.x; i < i1; i += 4 * kCdfBlock) {
-            if (i + 4 <= i1) {
-                const float4 v = *(const float4*)(l + i);
-                *(double2*)(e + i) = make_double2(exp_f64((double)v.x - m, c_exp.v), exp_f64((double)v.y - m, c_exp.v));
-                *(double2*)(e + i + 2) =
-                    make_double2(exp_f64((double)v.z - m, c_exp.v), exp_f64((double)v.w - m, c_exp.v));
-            } else {
-                for (uint32_t k = i; k < i1; k++) e[k] = exp_f64((double)l[k] - m, c_exp.v);
+    double* seg = a.seg + (size_t)row * segments(n);
+    const uint32_t lane = threadIdx.x % 64;
+    const bool vec = vec_row(l) && ((uintptr_t)e & 15) == 0;
+    for (uint32_t s0 = c * kChunk + threadIdx.x / 64 * kSegTerms; s0 < min(n, (c + 1) * kChunk);
+         s0 += kCdfBlock / 64 * kSegTerms) {
+        double sum = 0.0;
+        const uint32_t i = s0 + kTerms * lane;
+        if (vec && i + 4 <= n) {
+            const float4 v = *(const float4*)(l + i);
+            const double2 p = make_double2(exp_f64((double)v.x - m, c_exp.v), exp_f64((double)v.y - m, c_exp.v));
+            const double2 q = make_double2(exp_f64((double)v.z - m, c_exp.v), exp_f64((double)v.w - m, c_exp.v));
+            *(double2*)(e + i) = p;
+            *(double2*)(e + i + 2) = q;
+            sum = (p.x + p.y) + (q.x + q.y);
+        } else {
+            // a row that starts off 16 bytes (element s0 + lane + 64 k), or the row's last elements
+            const uint32_t first = vec ? i : s0 + lane, step = vec ? 1 : 64;
+            for (uint32_t k = 0; k < kTerms && first + k * step < n; k++) {
+                const double x = exp_f64((double)l[first + k * step] - m, c_exp.v);
+                e[first + k * step] = x;
+                sum += x;
             }
         }
-    } else {
-        for (uint32_t i = i0 + threadIdx.x; i < i1; i += kCdfBlock) e[i] = exp_f64((double)l[i] - m, c_exp.v);
+        sum = wave_incl_sum(sum);
+        if (lane == 63) seg[s0 / kSegTerms] = sum;
     }
 }
 
@@ -210,48 +249,37 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_exp(CdfArgs a) {
 // changes of the running sum s.  While s stays in [2^E, 2^(E+1)), every double there is a
 // multiple of u = 2^(E-52), s = T u with T < 2^53, and fl(s + x) = (T + a) u with
 // a = round(x / u), half to the side that makes T + a even, as long as T + a < 2^53 (else
-// the result leaves the binade and rounds on a coarser grid).  So a round takes 4096 terms,
-// each thread forms a for 4 of them, a block-wide prefix sum gives every T, and the first
-// term that is a NaN or takes T to 2^53 or beyond is an event: the terms before it are added
-// as the integer sum, the event itself with one real f64 add, and the next round starts after
-// it (on the new s's grid).  Halves (ties) need the parity of T, a prefix of one bit and a
-// reset (a tie leaves T even), formed beside the counts'.  They are not rare: an f32
-// probability 2^-29 of the sum or less has its last bit at or below half the sum's grid, and
-// most of a trained model's vocabulary lies there.  With each tie an event of its own, as
-// first built, 128 rows of 50,280 normal logits of standard deviations 1 to 4 took 3,768 us
-// here, against 93 us for the flat rows of an untrained model; with the parity prefix such rows'
-// whole CDF takes 178 us instead of 3,577.  Below 2^-1022 the grid is the subnormal spacing 2^-1074 with the same
-// rule.  A round without an event adds all its terms.  The result is the sequential sum
-// bit for bit (an event changes s exactly as the sequential add does; between events the
-// integer sum is exact).  The running sum of these rows stays below 2^24 (each term <= 1,
-// n < 2^24), so the grid is always finer than 1.  The grid counts are integer-valued f64
-// (no integer conversion is a single instruction for 64 bits): a sum of non-negative
-// integers is exact whenever its result is below 2^53, and rounding is monotone, so a sum
-// that reaches 2^53 still reads as >= 2^53 - the crossing test needs no more.  Prefixes
-// are formed by adding, never by subtracting, so that this holds for each of them.
+// the result leaves the binade and rounds on a coarser grid).  Halves (ties) need the parity
+// of T, a prefix of one bit and a reset (a tie leaves T even), formed beside the counts'.
+// They are not rare: an f32 probability 2^-29 of the sum or less has its last bit at or below
+// half the sum's grid, and most of a trained model's vocabulary lies there.  The grid counts
+// are integer-valued f64 (no integer conversion is a single instruction for 64 bits): a sum
+// of non-negative integers is exact whenever its result is below 2^53, and rounding is
+// monotone, so a sum that reaches 2^53 still reads as >= 2^53 - the crossing test needs no
+// more.  Prefixes are formed by adding, never by subtracting, so that this holds for each of
+// them.  Below 2^-1022 the grid is the subnormal spacing 2^-1074 with the same rule.
 //
-// The running sum of a row doubles about once per binade, and most of those crossings fall in
-// the row's first few hundred terms: a round each.  So the first kHead terms are added one by one, in order, by one
-// wave, from the registers of the lanes that loaded them (real f64 adds, the sequential sum
-// itself), and the rounds start after them.
-constexpr uint32_t kSumBlock = 1024;                 // threads of a row's workgroup
-constexpr uint32_t kSumWaves = kSumBlock / 64;
-constexpr uint32_t kTerms = 4;                       // terms per thread per round
-constexpr uint32_t kRound = kTerms * kSumBlock;      // terms per round
-constexpr uint32_t kHeadLanes = 64;                  // lanes of wave 0 whose terms form the head
-constexpr uint32_t kHead = kHeadLanes * kTerms;      // terms added one by one
-constexpr uint32_t kNoEvent = 0xffffffffu;
-static_assert(kHeadLanes <= 64 && kHead <= kRound, "the head lies in wave 0's terms of the first window");
-
-// A 64-bit value moved across lanes by DPP (each 32-bit half; lanes without a source
-// read 0): a few cycles, against an LDS round trip for a lane permute.
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const uint64_t b = as_u64(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
-    return as_f64(((uint64_t)hi << 32) | lo);
-}
+// So the row is cut into segments of 256 terms, a wave's.  k_cdf_exp's segment sums (any
+// order, a relative error of a few 2^-53) tell which binade s is in at each segment's two
+// ends; where it is the same one with 2^-30 to spare, the segment's whole count on that
+// binade's grid, with its ties' parity, is formed by any wave at any time (grid_count).  The
+// few segments where s may change binade, about one per doubling of s, are put into LDS
+// instead.  One wave then goes through the row (chain): it adds runs of counted segments as
+// one prefix sum of up to 64 counts, and takes the others in rounds (exact_segment): a prefix
+// sum of the terms' counts up to the first event (a NaN, or a term that takes T to 2^53 or
+// beyond), the event with one real f64 add, and the next round on the new s's grid.  A
+// counted segment is used only if s really is in its binade and its count keeps T below 2^53;
+// else it goes through the rounds too, so the result is the sequential sum bit for bit
+// whatever the segment sums say.  The first segment, where s doubles most often, is added term
+// by term.  The running sum of these rows stays below 2^24 (each term <= 1, n < 2^24), so
+// the grid is always finer than 1.
+//
+// 128 rows of 50,280 normal logits of standard deviations 1 to 4: 57 us, where 4,096 terms of
+// the whole workgroup a round in order (two barriers, 1.7 us each, about 46 rounds a row) took
+// 121; the whole CDF 175 -> 112.  Of a row, each sum: 1.8 us to classify, 7 to count (51 MB
+// of e over all rows at 7 TB/s; the second sum 8 to 17, by how many of its terms are ties), 10
+// to 14 in the chain, whose lone wave issues at a third of the vector rate: about 1.3 us for
+// each uncounted segment with the run before it.
 // The same value in every lane, made visibly uniform (scalar registers): the round loop's
 // control values come from LDS, and without this the compiler treats the loop as divergent
 // (exec masking, and copies of the prefetched terms that wait for their loads every round).
@@ -273,261 +301,366 @@ __device__ __forceinline__ double lane_f64(double v, int L) {
 // Lane L's copy of v for a wave-uniform L.
 __device__ __forceinline__ double lane_f64_at(double v, int L) { return lane_f64(v, (int)uni((uint32_t)L)); }
 
-// Inclusive prefix sum over the wave's 64 lanes: shifts by 1, 2, 4, 8 within each row of
-// 16 lanes, then the last lane of row 0 / 2 into rows 1 / 3 and lane 31 into rows 2 and 3.
-__device__ __forceinline__ double wave_incl_sum(double v) {
-    v += dpp_f64<0x111>(v);          // row_shr:1
-    v += dpp_f64<0x112>(v);          // row_shr:2
-    v += dpp_f64<0x114>(v);          // row_shr:4
-    v += dpp_f64<0x118>(v);          // row_shr:8
-    v += dpp_f64<0x142, 0xa>(v);     // row_bcast:15 into rows 1 and 3
-    v += dpp_f64<0x143, 0xc>(v);     // row_bcast:31 into rows 2 and 3
-    return v;
+// The members of a sequence of up to 64 (bit i: member i) that starts at an even T: members H
+// hold a tie and then leave the parity that P has for them, the others flip the parity by
+// their bit of P.  Bit i of the result: T is odd before member i.  All of it is scalar
+// arithmetic on one mask for the wave.
+__device__ __forceinline__ uint64_t odd_before(uint64_t H, uint64_t P) {
+    uint64_t x = P << 1;   // the flips of all members before, ties or not
+    x ^= x << 1;
+    x ^= x << 2;
+    x ^= x << 4;
+    x ^= x << 8;
+    x ^= x << 16;
+    x ^= x << 32;
+    // behind a tie only the flips from it on count: x of the last tie before is taken out, a bit
+    // that a carry spreads from the member behind that tie up to the next tie
+    const uint64_t other = ~H;
+    return x ^ ((((x & H) << 1) + other) ^ other);
 }
-
-// The parity of an integer-valued v in [0, 2^53].
-__device__ __forceinline__ uint32_t odd(double v) {
-    return (uint32_t)as_u64(v < 0x1p52 ? v + 0x1p52 : v) & (v < 0x1p53 ? 1u : 0u);
+// T's parity behind all of them.
+__device__ __forceinline__ uint32_t odd_behind(uint64_t H, uint64_t P) {
+    const uint64_t from = H != 0 ? ~0ull << (63 - __builtin_clzll(H)) : ~0ull;   // the last tie on
+    return (uint32_t)__builtin_popcountll(P & from) & 1u;
 }
+// Mask bit of the lane.
+__device__ __forceinline__ bool lane_in(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 
-// The parity of T behind the members `below` of a sequence that starts at an even T: member i
-// has a tie (bit i of H) and then leaves parity bit i of P, or flips the parity by bit i.
-__device__ __forceinline__ uint32_t parity_into(uint64_t H, uint64_t P, uint64_t below) {
-    const uint64_t h = H & below;
-    const uint64_t from = h != 0 ? ~0ull << (63 - __builtin_clzll(h)) : ~0ull;   // the last tie on
-    return (uint32_t)__builtin_popcountll(P & below & from) & 1u;
-}
+constexpr uint32_t kSumBlock = 1024;                 // threads of a row's workgroup
+constexpr uint32_t kSumWaves = kSumBlock / 64;
+constexpr uint32_t kWinSegs = 256;                   // segments of a window (65,536 terms)
+constexpr uint32_t kSlots = 24;                      // uncounted segments whose terms fit the LDS
+constexpr uint32_t kInFlight = 4;                    // segments a wave has requested ahead
+constexpr int kNoGrid = 0;                           // (every grid's scale is a positive power)
+static_assert(kWinSegs == 64 * kTerms, "wave 0 classifies kTerms segments a lane");
 
-// LDS of a round, double-buffered by round parity so that a round's writes never meet the
-// previous round's reads (two barriers per round).
 struct SumShared {
-    double part[2][kSumWaves];     // per-wave totals
-    uint32_t tie[2][kSumWaves];    // per-wave ties (wave_tie)
-    uint32_t first[2][kSumWaves];  // per-wave first event
-    double t_ev[2][kSumWaves];     // the grid count before that event
-    double x_ev[2][kSumWaves];     // that event's term
-    double s;                      // the head's or the fallback's result
-    double head[kHead];            // the head's terms in order
+    double terms[kSlots][kSegTerms];   // the first kSlots uncounted segments' terms, in order
+    double count[kWinSegs];            // a counted segment's grid count (grid_count)
+    int grid[kWinSegs];                // its grid 2^-grid, or kNoGrid
+    int slot[kWinSegs];                // an uncounted segment's place in terms, or kSlots or more
+    uint32_t tie[kWinSegs];            // its ties (grid_count)
+    double s;                          // the running sum after the window
 };
 
-// A barrier for the rounds' LDS traffic only: LDS operations complete (lgkmcnt 0), then
-// s_barrier.  __syncthreads would also wait for every global load in flight (vmcnt 0), and
-// the next window's terms are loaded while this window's rounds run.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // vmcnt and expcnt at their maxima, lgkmcnt 0
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+// A term's count on a grid: x / u to the nearest integer, halves to even, which is the
+// count's own rounding from an even T.  q = x / u must be below 2^52 (a larger one takes T past
+// the binade: T >= 2^52 before it, or 2^52 is the subnormal grid's end): q + 2^52 rounds to
+// an integer and shows its parity.
+struct GridTerm {
+    double a;       // the count
+    double d;       // q - a: a tie is +-1/2, and from an odd T its count is a + 2 d
+    uint32_t odd;   // the count's parity (bit 0)
+};
+__device__ __forceinline__ GridTerm grid_term(double q) {
+    GridTerm g;
+    const double m = q + 0x1p52;
+    g.a = m - 0x1p52;
+    g.d = q - g.a;
+    g.odd = (uint32_t)as_u64(m);
+    return g;
 }
 
+// +1 or -1 by d's sign in the lanes of the mask, else 0.
+__device__ __forceinline__ double unit_step(uint64_t mask, double d) {
+    const uint32_t hi = ((uint32_t)(as_u64(d) >> 32) & 0x80000000u) | 0x3ff00000u;
+    return as_f64((uint64_t)(lane_in(mask) ? hi : 0u) << 32);
+}
+
+// A wave's ties settled as far as they can be without the parity of T before the wave.  A tie
+// leaves an even T behind, so the parity a lane passes on is its own once it holds a tie, else
+// the incoming one flipped by its counts.  step[j]: the lanes whose term j is a tie from an odd
+// T (its count is a + 2 d); the wave's first tie (lane `first`, one bit; none: no tie) is
+// left as from an even T.
+struct WaveTies {
+    uint64_t step[kTerms], lead[kTerms];   // lead[j]: term j is its lane's first tie
+    uint64_t first;
+    uint64_t odd;    // T is odd before the lane's first tie if it is even before the wave
+    uint32_t behind;  // the parity of T behind the wave (without a tie: the flip)
+};
+__device__ __forceinline__ WaveTies wave_ties(const GridTerm (&g)[kTerms]) {
+    WaveTies w;
+    uint64_t x = 0, seen = 0, first_x = 0;   // x: parity since the lane's start or last tie
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) {
+        const uint64_t tie = __ballot(fabs(g[j].d) == 0.5);
+        w.lead[j] = tie & ~seen;
+        w.step[j] = tie & seen & x;
+        first_x |= w.lead[j] & x;
+        seen |= tie;
+        x = (x ^ __ballot((g[j].odd & 1u) != 0)) & ~tie;
+    }
+    w.odd = odd_before(seen, x) ^ first_x;
+    w.behind = odd_behind(seen, x);
+    w.first = seen & (0 - seen);
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) w.step[j] |= w.lead[j] & w.odd & ~w.first;
+    return w;
+}
+
+// Segment i's count on its grid, into sh.  Its bits in sh.tie: 1: it holds a tie; 2: T is odd
+// before the first one if it is even before the segment; 4: the parity of T behind it (without
+// a tie: the flip); 8: the first tie steps down from an odd T, not up.
+__device__ __forceinline__ void grid_count(const double (&fx)[kTerms], int ks, uint32_t i, int lane, SumShared& sh) {
+    const double scale = as_f64((uint64_t)(1023 + ks) << 52);
+    GridTerm g[kTerms];
+    bool any_tie = false;
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) {
+        g[j] = grid_term(fx[j] * scale);   // exact, or inf
+        any_tie |= fabs(g[j].d) == 0.5;
+    }
+    double mine = (g[0].a + g[1].a) + (g[2].a + g[3].a);
+    uint32_t ties = 0;
+    if (__ballot(any_tie) != 0) {
+        const WaveTies w = wave_ties(g);
+        uint64_t down = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kTerms; j++) {
+            mine += unit_step(w.step[j], g[j].d);
+            down |= w.lead[j] & __ballot(g[j].d < 0.0);
+        }
+        ties = 1u | ((w.odd & w.first) != 0 ? 2u : 0u) | w.behind << 2 | ((down & w.first) != 0 ? 8u : 0u);
+    }
+    const double total = wave_incl_sum(mine);
+    if (lane == 63) {
+        sh.count[i] = total;   // (NaN or not below 2^52 where a term is no count of the binade)
+        sh.tie[i] = ties != 0 ? ties : ((uint32_t)as_u64(total + 0x1p52) & 1u) << 2;
+    }
+}
+
+// s after the wave's 256 terms (lane L: terms L kTerms ..), by rounds.  Terms that are in s are
+// zeros from then on.
+__device__ double exact_segment(double (&fx)[kTerms], double s, int lane) {
+    for (;;) {
+        if (isnan(s)) return s;   // stays NaN (only NaN-ness is used downstream)
+        if (!(s < 0x1p52)) {
+            // a grid of 1 or coarser (not reached by these rows): the terms one by one
+            for (uint32_t i = 0; i < kSegTerms; i++) {
+                const uint32_t j = i % kTerms;
+                s += lane_f64_at(j == 0 ? fx[0] : j == 1 ? fx[1] : j == 2 ? fx[2] : fx[3], (int)(i / kTerms));
+            }
+            return s;
+        }
+        // the grid of the current binade: terms scale by 2^ks into units of it
+        const bool sub = s < 0x1p-1022;
+        const int ks = sub ? 1074 : 1075 - (int)(as_u64(s) >> 52);
+        const double top = sub ? 0x1p52 : 0x1p53;
+        const double T0 = ldexp(s, ks);   // exact and integer-valued: s is on the grid
+        GridTerm g[kTerms];
+        bool bad[kTerms];   // NaN, inf or certainly past the binade: an event
+        bool any_tie = false;
+#pragma unroll
+        for (uint32_t j = 0; j < kTerms; j++) {
+            const double q = ldexp(fx[j], ks);   // exact, or +inf past the double range
+            bad[j] = !(q < 0x1p52);
+            g[j] = grid_term(bad[j] ? 0.0 : q);
+            any_tie |= fabs(g[j].d) == 0.5;
+        }
+        if (__ballot(any_tie) != 0) {
+            const WaveTies w = wave_ties(g);
+            const bool t_odd = ((uint32_t)as_u64(sub ? T0 + 0x1p52 : T0) & 1u) != 0;
+            const uint64_t first = ((w.odd & w.first) != 0) != t_odd ? w.first : 0;   // if it steps
+#pragma unroll
+            for (uint32_t j = 0; j < kTerms; j++) g[j].a += unit_step(w.step[j] | (w.lead[j] & first), g[j].d);
+        }
+        double c[kTerms];   // the lane's inclusive prefix
+        double mine = 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < kTerms; j++) {
+            mine += g[j].a;
+            c[j] = mine;
+        }
+        const double incl = wave_incl_sum(mine);
+        const double base = T0 + dpp_f64<0x138>(incl);   // wave_shr:1 (lane 0 reads 0)
+        // the lane's first term that is bad or takes T to the top of the binade
+        bool hit = false;
+        uint32_t at = 0;
+        double T_ev = 0.0, x_ev = 0.0;
+#pragma unroll
+        for (int j = (int)kTerms - 1; j >= 0; j--) {
+            const bool h = bad[j] || base + c[j] >= top;
+            hit |= h;
+            at = h ? (uint32_t)j : at;
+            T_ev = h ? (j > 0 ? base + c[j - 1] : base) : T_ev;
+            x_ev = h ? fx[j] : x_ev;
+        }
+        const uint64_t has = __ballot(hit);
+        if (has == 0) return uni(ldexp(T0 + lane_f64(incl, 63), -ks));   // no event: T0 + total < top
+        const int src = (int)uni((uint32_t)__builtin_ctzll(has));
+        s = uni(ldexp(lane_f64(T_ev, src), -ks) + lane_f64(x_ev, src));
+        const uint32_t done = (uint32_t)src * kTerms + (uint32_t)__builtin_amdgcn_readlane((int)at, src);
+#pragma unroll
+        for (uint32_t j = 0; j < kTerms; j++) fx[j] = (uint32_t)lane * kTerms + j <= done ? 0.0 : fx[j];
+    }
+}
+
+// Terms kTerms lane .. of the segment that starts at k0; past the row's end 0, which no sum of
+// the row tells from nothing (s is +0 or more once it holds a term).
 template <class F>
-__device__ double exact_seq_sum(const double* __restrict__ e, uint32_t n, double s, F f, SumShared& sh) {
-    const uint32_t t = threadIdx.x;
-    const int lane = t % 64, w = t / 64;
-    // The window's terms stay in registers (thread t: terms t kTerms .. + kTerms - 1).
-    // The next window's terms are requested before this window's first round and arrive
-    // while its rounds run; the rounds wait only for LDS.
-    uint32_t par = 0;
-    double nx[kTerms];
+__device__ __forceinline__ void seg_terms(uint32_t n, uint32_t k0, int lane, F f, const double (&raw)[kTerms],
+                                          double (&fx)[kTerms]) {
+    if (k0 + kSegTerms <= n) {
 #pragma unroll
-    for (uint32_t j = 0; j < kTerms; j++) nx[j] = e[min(t * kTerms + j, n - 1)];
-    for (uint32_t k0 = 0; k0 < n; k0 += kRound) {
-        double fx[kTerms];
-        __builtin_amdgcn_s_waitcnt(0);
+        for (uint32_t j = 0; j < kTerms; j++) fx[j] = f(raw[j]);
+        return;
+    }
 #pragma unroll
-        for (uint32_t j = 0; j < kTerms; j++) fx[j] = f(nx[j]);
-        if (k0 + kRound < n) {
+    for (uint32_t j = 0; j < kTerms; j++) fx[j] = k0 + (uint32_t)lane * kTerms + j < n ? f(raw[j]) : 0.0;
+}
+__device__ __forceinline__ void seg_load(const double* __restrict__ e, uint32_t n, uint32_t k0, int lane,
+                                         double (&raw)[kTerms]) {
+    if (k0 + kSegTerms <= n && ((uintptr_t)(e + k0) & 15) == 0) {
+        const double2* p = (const double2*)(e + k0 + (uint32_t)lane * kTerms);
+        const double2 v = p[0], w = p[1];
+        raw[0] = v.x, raw[1] = v.y, raw[2] = w.x, raw[3] = w.y;
+        return;
+    }
 #pragma unroll
-            for (uint32_t j = 0; j < kTerms; j++) nx[j] = e[min(k0 + kRound + t * kTerms + j, n - 1)];
+    for (uint32_t j = 0; j < kTerms; j++) raw[j] = e[min(k0 + (uint32_t)lane * kTerms + j, n - 1)];
+}
+
+// Which of the window's m segments lie in one binade, and the others' slots in order (wave 0).
+// The segment sums are scaled by `scale`; s is the running sum before the window.
+__device__ void classify(const double* __restrict__ seg, uint32_t m, double scale, double s, int lane, SumShared& sh) {
+    double v[kTerms];
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) v[j] = seg[min((uint32_t)lane * kTerms + j, m - 1)] * scale;
+    const double incl = wave_incl_sum((v[0] + v[1]) + (v[2] + v[3]));
+    double at = s + dpp_f64<0x138>(incl);
+    int grid[kTerms];
+    uint32_t place = 0;   // uncounted segments of the lanes before
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) {
+        // (exponents from 2^-900 to 2^51: the grid's scale is a normal double; NaN and inf: 2047)
+        const uint32_t lo = (uint32_t)(as_u64(at * (1.0 - 0x1p-30)) >> 52);
+        at += v[j];
+        const uint32_t hi = (uint32_t)(as_u64(at * (1.0 + 0x1p-30)) >> 52);
+        grid[j] = lo == hi && lo >= 1023 - 900 && lo < 1023 + 52 ? 1075 - (int)lo : kNoGrid;
+        const uint64_t un = __ballot((uint32_t)lane * kTerms + j < m && grid[j] == kNoGrid);
+        place += (uint32_t)__builtin_popcountll(un & ((1ull << lane) - 1));
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) {
+        const uint32_t i = (uint32_t)lane * kTerms + j;
+        if (i < m) {
+            sh.grid[i] = grid[j];
+            sh.slot[i] = (int)place;
+            place += grid[j] == kNoGrid ? 1u : 0u;
         }
-        // rounds over this window: after an event the rest of the window is re-gridded
-        uint32_t from = 0;   // first term of the window not yet in s
-        if (k0 == 0 && n >= kHead) {
-            // the head: terms 0 .. kHead - 1 in order.  Wave 0 holds them (lane L: terms
-            // L kTerms ..); it stores them to LDS in order and every lane reads them back
-            // (same address: a broadcast) into one chain of adds.
-            if (w == 0) {
-#pragma unroll
-                for (uint32_t j = 0; j < kTerms; j++)
-                    if (lane < (int)kHeadLanes) sh.head[lane * kTerms + j] = fx[j];
-                __builtin_amdgcn_s_waitcnt(0xc07f);   // this wave's LDS stores done
-                __builtin_amdgcn_wave_barrier();
-                double acc = s;
+    }
+}
+
+// s after the window's m segments (wave 0).
+template <class F>
+__device__ double chain(const double* __restrict__ e, uint32_t n, uint32_t k0, uint32_t m, double s, int lane, F f,
+                        const SumShared& sh) {
+    uint32_t i = 0;
+    uint32_t slots = 0;   // uncounted segments before segment i
+    if (k0 == 0) {
+        // the row's first segment in order (classify leaves s = 0 without a grid and gives it
+        // the first slot): every lane reads the terms back as broadcasts into one chain of adds
 #pragma unroll 2
-                for (uint32_t i = 0; i < kHead; i += 16) {
-                    double v[16];
+        for (uint32_t t = 0; t < kSegTerms; t += 16) {
+            double v[16];
 #pragma unroll
-                    for (uint32_t k = 0; k < 16; k++) v[k] = sh.head[i + k];
+            for (uint32_t k = 0; k < 16; k++) v[k] = sh.terms[0][t + k];
 #pragma unroll
-                    for (uint32_t k = 0; k < 16; k++) acc += v[k];
-                }
-                if (lane == 0) sh.s = acc;
-            }
-            lds_barrier();
-            s = uni(sh.s);
-            from = kHead;
-            lds_barrier();   // sh.s and sh.head are read before any later write to them
+            for (uint32_t k = 0; k < 16; k++) s += v[k];
         }
-        while (from < kRound && k0 + from < n) {
-            if (isnan(s)) return s;   // stays NaN (only NaN-ness is used downstream)
-            if (!(s < 0x1p52)) {
-                // a grid of 1 or coarser (not reached by these rows): finish in order on one thread
-                __syncthreads();
-                if (t == 0) {
-                    for (uint32_t i = k0 + from; i < n; i++) s += f(e[i]);
-                    sh.s = s;
-                }
-                __syncthreads();
-                return uni(sh.s);
-            }
-            // the grid of the current binade: terms scale by 2^ks into units of it
-            int ks;
-            double top;
-            if (s < 0x1p-1022) {
-                ks = 1074;
-                top = 0x1p52;
-            } else {
-                ks = 52 - ilogb(s);
-                top = 0x1p53;
-            }
-            const double T0 = ldexp(s, ks);   // exact and integer-valued: s is on the grid
-            double a[kTerms];   // grid counts; 0 for events and for terms outside the round
-            double c[kTerms];   // this thread's inclusive prefix of them
-            bool live[kTerms];
-            bool tie[kTerms];   // x / u halfway between two counts: a holds the lower one
-            uint32_t ev = kNoEvent;   // this thread's first NaN or term past the binade (index within the window)
-            bool any_tie = false;
-            // (straight-line: selects, no branches per term)
+        s = uni(s);
+        i = 1;
+        slots = 1;
+    }
+    while (i < m) {
+        if (isnan(s)) return s;
+        // the next uncounted segment's terms, requested before the counts are added up
+        double fx[kTerms];
 #pragma unroll
-            for (uint32_t j = 0; j < kTerms; j++) {
-                const uint32_t r = t * kTerms + j;
-                live[j] = r >= from && k0 + r < n;
-                const double q = ldexp(fx[j], ks);     // exact, or +inf past the double range
-                // round half to even: every non-tie rounds as fl(s + x) does; q - m is exact
-                const double m = rint(q);
-                const bool bad = !(q < 0x1p53);        // NaN, inf or certainly past the binade
-                ev = (live[j] && bad && ev == kNoEvent) ? r : ev;
-                tie[j] = live[j] && !bad && fabs(q - m) == 0.5;
-                any_tie |= tie[j];
-                a[j] = (live[j] && !bad) ? (tie[j] ? floor(q) : m) : 0.0;
+        for (uint32_t j = 0; j < kTerms; j++) fx[j] = sh.terms[min(slots, kSlots - 1)][(uint32_t)lane * kTerms + j];
+        const int ks = s < 0x1p-1022 || !(s < 0x1p52) ? kNoGrid - 1 : 1075 - (int)(as_u64(s) >> 52);
+        // the counted segments of s's binade from here on, up to 64
+        const uint32_t i0 = i, at = min(i + (uint32_t)lane, m - 1);
+        const int grid = sh.grid[at];
+        const double count = sh.count[at];
+        const uint32_t ties = sh.tie[at];
+        const uint64_t off = ~__ballot(i + (uint32_t)lane < m && grid == ks);
+        const int run = off != 0 ? __builtin_ctzll(off) : 64;
+        if (run > 0) {
+            double c = lane < run ? count : 0.0;
+            const uint32_t t = lane < run ? ties : 0u;
+            const double T0 = ldexp(s, ks);
+            const uint64_t H = __ballot((t & 1u) != 0);
+            if (H != 0) {
+                // each segment's first tie, from the parity of T before that segment
+                const uint64_t t_odd = ((uint32_t)as_u64(T0) & 1u) != 0 ? ~0ull : 0ull;
+                const uint64_t in = odd_before(H, __ballot((t & 4u) != 0)) ^ (t_odd & ((H & (0 - H)) | ((H & (0 - H)) - 1)));
+                const uint64_t step = H & (in ^ __ballot((t & 2u) != 0));
+                c += lane_in(step) ? ((t & 8u) != 0 ? -1.0 : 1.0) : 0.0;
             }
-            // A tie rounds to the even count, so it needs the parity of T before it and leaves
-            // an even T behind: the parity a thread (a wave) passes on is its own once it holds
-            // a tie, else the incoming one flipped by its counts.  The lanes' two bits are
-            // combined from ballots, so every tie of a wave but its first is settled here and
-            // the first one (lane tie_lane, term tie_j) with the waves' own two bits below.
-            uint32_t wave_tie = 0;        // bit 0: the wave holds a tie; bit 1: the first one's
-                                          // rounding up if T is even before the wave; bit 2: parity out
-            int tie_lane = 64;
-            uint32_t tie_j = kTerms;
-            if (__ballot(any_tie) != 0) {
-                uint32_t x = 0, first_up = 0;   // parity since the thread's start or last tie
-                bool seen = false;
-#pragma unroll
-                for (uint32_t j = 0; j < kTerms; j++) {
-                    const uint32_t up = x ^ odd(a[j]);
-                    if (tie[j] && !seen) {
-                        first_up = up;
-                        tie_j = j;
-                    } else if (tie[j]) {
-                        a[j] += (double)up;
-                    }
-                    seen |= tie[j];
-                    x = tie[j] ? 0u : up;
-                }
-                const uint64_t H = __ballot(seen), P = __ballot(x != 0);
-                const uint64_t below = (1ull << lane) - 1;
-                const uint32_t in = parity_into(H, P, below);   // from an even T before the wave
-                tie_lane = (int)__builtin_ctzll(H);
-                if (seen && lane != tie_lane) {
-#pragma unroll
-                    for (uint32_t j = 0; j < kTerms; j++) a[j] += j == tie_j ? (double)(in ^ first_up) : 0.0;
-                }
-                wave_tie = 1u | (uint32_t)__builtin_amdgcn_readlane((int)(in ^ first_up), tie_lane) << 1 |
-                           parity_into(H, P, ~0ull) << 2;
-            }
-            double mine = 0.0;
-#pragma unroll
-            for (uint32_t j = 0; j < kTerms; j++) {
-                mine += a[j];
-                c[j] = mine;
-            }
-            // workgroup prefix of the grid counts: the lane's exclusive prefix in its wave
-            // (the inclusive prefix of the lane before it), then the waves before it
-            const double incl = wave_incl_sum(mine);
-            if (lane == 63) {
-                sh.part[par][w] = incl;
-                sh.tie[par][w] = (wave_tie & 1u) ? wave_tie : odd(incl) << 2;
-            }
-            double before = dpp_f64<0x138>(incl);   // wave_shr:1 (lane 0 reads 0)
-            lds_barrier();
-            // lanes 0 .. kSumWaves - 1 read one wave's total each; their inclusive prefix gives
-            // the waves before this one and the workgroup's total
-            double wp = lane < (int)kSumWaves ? sh.part[par][lane] : 0.0;
-            const uint32_t wt = lane < (int)kSumWaves ? sh.tie[par][lane] : 0u;
-            const uint64_t Hw = __ballot((wt & 1u) != 0);
-            if (Hw != 0) {
-                // each wave's first tie, from the parity of T before that wave
-                const uint64_t Pw = __ballot((wt & 4u) != 0), below = (1ull << lane) - 1;
-                const bool settled = (Hw & below) != 0;
-                const uint32_t in = parity_into(Hw, Pw, below) ^ (settled ? 0u : odd(T0));
-                const double up = (wt & 1u) ? (double)(in ^ ((wt >> 1) & 1u)) : 0.0;
-                wp += up;
-                const double mine_up = lane_f64_at(up, w);
-                before += lane > tie_lane ? mine_up : 0.0;
-#pragma unroll
-                for (uint32_t j = 0; j < kTerms; j++) c[j] += (lane == tie_lane && j >= tie_j) ? mine_up : 0.0;
-            }
-            wp += dpp_f64<0x111>(wp);   // row_shr:1, 2, 4, 8 within lanes 0 .. 15
-            wp += dpp_f64<0x112>(wp);
-            wp += dpp_f64<0x114>(wp);
-            wp += dpp_f64<0x118>(wp);
-            static_assert(kSumWaves <= 16, "the wave totals fit one DPP row");
-            const double waves = w > 0 ? lane_f64(wp, (int)uni((uint32_t)(w - 1))) : 0.0;
-            const double total = lane_f64(wp, (int)kSumWaves - 1);
-            // crossings: the first term whose add takes T to the top of the binade, or this
-            // thread's first NaN or term past it, whichever comes first (lowest j wins)
-            const double base = (T0 + waves) + before;
-            uint32_t evn = kNoEvent;
-            double T_ev = 0.0, x_ev = 0.0;
-#pragma unroll
-            for (int j = (int)kTerms - 1; j >= 0; j--) {
-                const uint32_t r = t * kTerms + (uint32_t)j;
-                const bool hit = live[j] && (r == ev || (r < ev && base + c[j] >= top));
-                evn = hit ? r : evn;
-                T_ev = hit ? (j > 0 ? base + c[j - 1] : base) : T_ev;
-                x_ev = hit ? fx[j] : x_ev;
-            }
-            ev = evn;
-            // the wave's first event sits in its lowest lane that has one (lanes hold
-            // consecutive terms)
-            const uint64_t has = __ballot(ev != kNoEvent);
-            if (lane == 0) sh.first[par][w] = kNoEvent;
-            if (has != 0) {
-                const int src = __builtin_ctzll(has);
-                if (lane == src) {
-                    sh.first[par][w] = ev;
-                    sh.t_ev[par][w] = T_ev;
-                    sh.x_ev[par][w] = x_ev;
-                }
-            }
-            lds_barrier();
-            // the round's first event is the first event of the lowest wave that has one
-            const uint32_t fv = lane < (int)kSumWaves ? sh.first[par][lane] : kNoEvent;
-            const uint64_t hasw = __ballot(fv != kNoEvent);
-            if (hasw == 0) {
-                // no event: the window's remaining terms are the grid sum (T0 + total < 2^53)
-                s = uni(ldexp(T0 + total, -ks));
-                from = kRound;
-            } else {
-                // the event's add, done by every thread on the same operands
-                const int fw = (int)uni((uint32_t)__builtin_ctzll(hasw));
-                const double tv = lane < (int)kSumWaves ? sh.t_ev[par][lane] : 0.0;
-                const double xv = lane < (int)kSumWaves ? sh.x_ev[par][lane] : 0.0;
-                s = uni(ldexp(lane_f64(tv, fw), -ks) + lane_f64(xv, fw));
-                from = (uint32_t)__builtin_amdgcn_readlane((int)fv, fw) + 1;
-            }
-            par ^= 1u;
+            const double T = T0 + wave_incl_sum(c);
+            const uint64_t past = __ballot(lane < run && !(T < 0x1p53));
+            const int take = past != 0 ? __builtin_ctzll(past) : run;
+            if (take > 0) s = uni(ldexp(lane_f64_at(T, take - 1), -ks));
+            i += (uint32_t)take;
+            if (take == 64 || i >= m) continue;
         }
+        // segment i: lane i - i0's, whose grid is not s's or whose count takes T to the top
+        const bool counted = __builtin_amdgcn_readlane(grid, (int)uni(i - i0)) != kNoGrid;
+        if (counted || slots >= kSlots) {
+            double raw[kTerms];
+            seg_load(e, n, k0 + i * kSegTerms, lane, raw);
+            seg_terms(n, k0 + i * kSegTerms, lane, f, raw, fx);
+        }
+        slots += counted ? 0u : 1u;
+        s = exact_segment(fx, s, lane);
+        i++;
+    }
+    return s;
+}
+
+// The sequential sum s + f(e[0]) + f(e[1]) + ... of the row; f(x) is about x * scale.
+template <class F>
+__device__ double exact_seq_sum(const double* __restrict__ e, const double* __restrict__ seg, uint32_t n, double s,
+                                double scale, F f, SumShared& sh) {
+    const int lane = threadIdx.x % 64;
+    const uint32_t w = uni(threadIdx.x / 64);
+    for (uint32_t k0 = 0; k0 < n; k0 += kWinSegs * kSegTerms) {
+        const uint32_t m = min(kWinSegs, segments(n - k0));
+        // wave w: segments w, w + kSumWaves, ..., kInFlight requested ahead
+        double nx[kInFlight][kTerms];
+#pragma unroll
+        for (uint32_t d = 0; d < kInFlight; d++) seg_load(e, n, k0 + (w + d * kSumWaves) * kSegTerms, lane, nx[d]);
+        if (w == 0) classify(seg + k0 / kSegTerms, m, scale, s, lane, sh);
+        __syncthreads();
+        for (uint32_t i0 = w; i0 < m; i0 += kInFlight * kSumWaves) {
+#pragma unroll
+            for (uint32_t d = 0; d < kInFlight; d++) {
+                const uint32_t i = i0 + d * kSumWaves;
+                double fx[kTerms];
+                seg_terms(n, k0 + i * kSegTerms, lane, f, nx[d], fx);
+                if (i + kInFlight * kSumWaves < m) seg_load(e, n, k0 + (i + kInFlight * kSumWaves) * kSegTerms, lane, nx[d]);
+                if (i >= m) continue;
+                const int ks = __builtin_amdgcn_readfirstlane(sh.grid[i]);
+                if (ks != kNoGrid) {
+                    grid_count(fx, ks, i, lane, sh);
+                    continue;
+                }
+                const int slot = __builtin_amdgcn_readfirstlane(sh.slot[i]);
+                if (slot < (int)kSlots) {
+#pragma unroll
+                    for (uint32_t j = 0; j < kTerms; j++) sh.terms[slot][(uint32_t)lane * kTerms + j] = fx[j];
+                }
+            }
+        }
+        __syncthreads();
+        if (w == 0) {
+            s = chain(e, n, k0, m, s, lane, f, sh);
+            if (lane == 0) sh.s = s;
+        }
+        __syncthreads();
+        s = uni(sh.s);
+        // (the next write to sh.s comes after the next window's or sum's barriers)
     }
     return s;
 }
@@ -536,9 +669,11 @@ __global__ __launch_bounds__(kSumBlock) void k_cdf_sums(CdfArgs a) {
     __shared__ SumShared sh;
     const uint32_t row = blockIdx.x, n = a.n;
     const double* e = a.e + (size_t)row * n;
-    const double s = uni(exact_seq_sum(e, n, 0.0, [](double v) { return v; }, sh));
+    const double* seg = a.seg + (size_t)row * segments(n);
+    const double s = exact_seq_sum(e, seg, n, 0.0, 1.0, [](double v) { return v; }, sh);
     const double inv_sum = 1.0 / s;
-    const double sp = exact_seq_sum(e, n, -0.0, [inv_sum](double v) { return (double)prob_of(v, inv_sum); }, sh);
+    const double sp = exact_seq_sum(e, seg, n, -0.0, inv_sum,
+                                    [inv_sum](double v) { return (double)prob_of(v, inv_sum); }, sh);
     if (threadIdx.x == 0) {
         a.sums[2 * row] = s;
         a.sums[2 * row + 1] = sp;
@@ -684,7 +819,8 @@ uint32_t cdf_chunks(uint32_t n) { return (n + kChunk - 1) / kChunk; }
 }  // namespace
 
 size_t cdf_scratch_bytes(uint32_t rows, uint32_t n) {
-    return (size_t)rows * n * 8 + (size_t)rows * 16 + (size_t)rows * cdf_chunks(n) * sizeof(ChunkPart);
+    return (size_t)rows * n * 8 + (size_t)rows * 16 + (size_t)rows * segments(n) * 8 +
+           (size_t)rows * cdf_chunks(n) * sizeof(ChunkPart);
 }
 
 hipError_t cdf_launch(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* cdf, hipStream_t st) {
@@ -692,8 +828,9 @@ hipError_t cdf_launch(const float* logits, uint32_t rows, uint32_t n, void* scra
     const uint32_t chunks = cdf_chunks(n);
     double* e = (double*)scratch;
     double* sums = e + (size_t)rows * n;
-    ChunkPart* part = (ChunkPart*)(sums + 2 * (size_t)rows);
-    CdfArgs a{logits, rows, n, chunks, e, sums, part, cdf};
+    double* seg = sums + 2 * (size_t)rows;
+    ChunkPart* part = (ChunkPart*)(seg + (size_t)rows * segments(n));
+    CdfArgs a{logits, rows, n, chunks, e, sums, seg, part, cdf};
     const dim3 grid(chunks, rows);
     k_cdf_max<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_exp<<<grid, dim3(kCdfBlock), 0, st>>>(a);

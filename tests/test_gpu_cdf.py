@@ -103,8 +103,25 @@ def tie_rows():
     return rows
 
 
-def test_device_cdf_equals_host_cdf_on_rows_of_ties(backend):
-    for name, row in tie_rows():
+def segment_rows():
+    """Rows at the edges of the sums' segments (256 terms) and windows (65,536), and rows whose
+    running sum changes binade in every segment or in more of them than have room in LDS."""
+    rng = np.random.default_rng(5)
+    rows = [("normal", (rng.standard_normal(n) * 2).astype(np.float32))
+            for n in (511, 512, 513, 65535, 65537, 65792, 131072, 131073, 200001)]
+    for n, low in ((50280, -600.0), (50281, -60.0), (70000, -720.0)):
+        rows.append((f"rising{low:g}", np.linspace(low, 0.0, n, dtype=np.float32)))
+        rows.append((f"falling{low:g}", np.linspace(0.0, low, n, dtype=np.float32)))
+    t = np.full(66000, -30.0, np.float32)
+    t[40000:] = -5.0
+    t[65540] = 0.0
+    rows.append(("steps", t))
+    return rows
+
+
+@pytest.mark.parametrize("rows", [tie_rows, segment_rows])
+def test_device_cdf_equals_host_cdf_on_rows_of_ties(backend, rows):
+    for name, row in rows():
         n = row.size
         d_l, d_c = hip.DeviceBuffer.from_array(row), hip.DeviceBuffer((n + 1) * 4)
         try:

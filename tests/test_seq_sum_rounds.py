@@ -171,3 +171,80 @@ def test_a_missed_tie_is_caught():
 
     assert not same(ties_up(x, 0.0), sequential(x, 0.0))
     assert same(rounds_sum(x, 0.0), sequential(x, 0.0))
+
+
+# ---- segments: counted apart on a guessed binade, then chained (k_cdf_sums) ----
+
+def seg_count(seg, ks):
+    """A segment's count on the grid 2^-ks without the parity before it: (count with the first
+    tie rounded down, first tie's rounding up from an even T or None, parity behind)."""
+    total, x, first_up = 0, 0, None
+    for v in seg:
+        q = ldexp_inf(v, ks)
+        if not q < 2.0 ** 53:
+            return 1 << 53, None, 0      # a NaN or past the binade: never used
+        m = math.floor(q)
+        x ^= m & 1
+        total += m
+        if q - m == 0.5:
+            if first_up is None:
+                first_up = x
+            else:
+                total += x
+            x = 0
+        elif q - m > 0.5:
+            total += 1
+            x ^= 1
+    return total, first_up, x
+
+
+def segments_sum(x, s0, seg=16, guess=None):
+    """The device's steps: each segment counted on the binade that `guess` (the running sum
+    before each segment and after the last, any approximation) puts its two ends in; the chain
+    uses a count where s is in that binade and stays below its top, else the rounds."""
+    x = [float(v) for v in x]
+    segs = [x[k:k + seg] for k in range(0, len(x), seg)]
+    if guess is None:
+        guess = np.concatenate([[0.0], np.cumsum([math.fsum(v) for v in segs])])
+    counts = []
+    for k, v in enumerate(segs):
+        lo, hi = guess[k] * (1 - 2.0 ** -30), guess[k + 1] * (1 + 2.0 ** -30)
+        ok = 2.0 ** -1021 <= lo and hi < 2.0 ** 52 and math.frexp(lo)[1] == math.frexp(hi)[1]
+        ks = 53 - math.frexp(lo)[1] if ok else None
+        counts.append((ks, *(seg_count(v, ks) if ok else (0, None, 0))))
+    s, used = float(s0), 0
+    for v, (ks, total, first_up, _) in zip(segs, counts):
+        if ks is not None and not math.isnan(s) and 2.0 ** -1022 <= s and ks == 53 - math.frexp(s)[1]:
+            T0 = int(math.ldexp(s, ks))
+            T = T0 + total + (0 if first_up is None else first_up ^ (T0 & 1))
+            if T < 1 << 53:
+                s, used = math.ldexp(float(T), -ks), used + 1
+                continue
+        s = rounds_sum(v, s, window=seg)
+    return s, used
+
+
+@pytest.mark.parametrize("seg", [1, 16, 256])
+@pytest.mark.parametrize("spread", [0.0, 1.0, 4.0, 60.0])
+def test_segments_counted_apart(seg, spread):
+    rng = np.random.default_rng([seg, int(spread)])
+    logits = rng.standard_normal(5000) * spread
+    e = np.exp(logits - logits.max())
+    s, used = segments_sum(e, 0.0, seg)
+    assert same(s, sequential(e, 0.0)) and used > 0
+    p = (e * (1.0 / s)).astype(np.float32).astype(np.float64)
+    s, _ = segments_sum(p, -0.0, seg)
+    assert same(s, sequential(p, -0.0))
+    half = np.tile([2.0 ** -53, 3 * 2.0 ** -53, 2.0 ** -52], 700)     # ties beside a sum of 1
+    t = np.concatenate([[1.0], half])
+    assert same(segments_sum(t, 0.0, seg)[0], sequential(t, 0.0))
+
+
+def test_segments_with_a_wrong_guess_or_a_nan():
+    rng = np.random.default_rng(3)
+    x = np.exp(rng.standard_normal(4000) * 2)
+    right = np.concatenate([[0.0], np.cumsum([math.fsum(x[k:k + 16]) for k in range(0, 4000, 16)])])
+    for wrong in (right * 2, right / 2, right * 0, right * np.nan, np.full(len(right), 7.0), right[::-1]):
+        assert same(segments_sum(x, 0.0, 16, wrong)[0], sequential(x, 0.0))
+    x[1234] = np.nan
+    assert math.isnan(segments_sum(x, 0.0, 16, right)[0])
