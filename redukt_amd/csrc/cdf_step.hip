@@ -98,13 +98,6 @@ __device__ double exp_f64(double x, const uint64_t* __restrict__ table) {
     return scale + scale * tmp;
 }
 
-// Rust's `f as u64`: truncation toward zero, NaN -> 0, saturating at both ends.
-__device__ __forceinline__ uint64_t sat_u64(double v) {
-    if (!(v > 0.0)) return 0;
-    if (v >= 18446744073709551616.0) return ~0ULL;
-    return (uint64_t)v;
-}
-
 // One row's f32 probability, the host's p[i] = float(e[i] * inv_sum).
 __device__ __forceinline__ float prob_of(double e, double inv_sum) { return (float)(e * inv_sum); }
 
@@ -118,18 +111,16 @@ struct ChunkPart {
     double max;        // the chunk's max (NaN loses; -inf if none)
     uint64_t used;     // sum of the chunk's extra frequencies
     uint64_t best;     // (largest frequency << 32) | its last index
-    uint32_t total;    // sum of the chunk's frequencies before the fix-up (u32, wrapping)
-    uint32_t pad;
 };
 
 struct CdfArgs {
     const float* logits;   // [rows][n]
     uint32_t rows, n, chunks;
     double* e;             // [rows][n] scratch: exp(logit - max)
-    double* sums;          // [rows][2] scratch: sum of e, sum of the probabilities
+    double* sums;          // [rows] scratch: the sum of the probabilities
     double* seg;           // [rows][segments] scratch: sum of each kSegTerms elements of e, in any order
     ChunkPart* part;       // [rows][chunks] scratch
-    uint32_t* cdf;         // [rows][n + 1]
+    uint32_t* cdf;         // [rows][n + 1]; k_cdf_sums leaves probability i's bits in element i + 1
 };
 
 // Block-wide reductions over kCdfBlock threads (four waves of 64).
@@ -274,9 +265,9 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_exp(CdfArgs a) {
 // by term.  The running sum of these rows stays below 2^24 (each term <= 1, n < 2^24), so
 // the grid is always finer than 1.
 //
-// 128 rows of 50,280 normal logits of standard deviations 1 to 4: 57 us, where 4,096 terms of
-// the whole workgroup a round in order (two barriers, 1.7 us each, about 46 rounds a row) took
-// 121; the whole CDF 175 -> 112.  Of a row, each sum: 1.8 us to classify, 7 to count (51 MB
+// 128 rows of 50,280 normal logits of standard deviations 1 to 4: 57 us (67 with the shares
+// after the sums), where 4,096 terms of the whole workgroup a round in order (two barriers,
+// 1.7 us each, about 46 rounds a row) took 121; the whole CDF 175 -> 112.  Of a row, each sum: 1.8 us to classify, 7 to count (51 MB
 // of e over all rows at 7 TB/s; the second sum 8 to 17, by how many of its terms are ties), 10
 // to 14 in the chain, whose lone wave issues at a third of the vector rate: about 1.3 us for
 // each uncounted segment with the run before it.
@@ -619,10 +610,29 @@ __device__ double chain(const double* __restrict__ e, uint32_t n, uint32_t k0, u
     return s;
 }
 
-// The sequential sum s + f(e[0]) + f(e[1]) + ... of the row; f(x) is about x * scale.
-template <class F>
+// f's terms as f32 bits to p (lane L: kTerms L ..).
+__device__ __forceinline__ void seg_store(uint32_t* p, uint32_t n, uint32_t k0, int lane, const double (&fx)[kTerms]) {
+    struct __attribute__((packed, aligned(4))) U4 {
+        uint32_t v[kTerms];
+    };
+    U4 u;
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) u.v[j] = __float_as_uint((float)fx[j]);
+    const uint32_t i = k0 + (uint32_t)lane * kTerms;
+    if (k0 + kSegTerms <= n) {
+        *(U4*)(p + i) = u;
+        return;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++)
+        if (i + j < n) p[i + j] = u.v[j];
+}
+
+// The sequential sum s + f(e[0]) + f(e[1]) + ... of the row; f(x) is about x * scale.  P: the
+// terms, which are f32 values, also go to p.
+template <bool P, class F>
 __device__ double exact_seq_sum(const double* __restrict__ e, const double* __restrict__ seg, uint32_t n, double s,
-                                double scale, F f, SumShared& sh) {
+                                double scale, F f, uint32_t* p, SumShared& sh) {
     const int lane = threadIdx.x % 64;
     const uint32_t w = uni(threadIdx.x / 64);
     for (uint32_t k0 = 0; k0 < n; k0 += kWinSegs * kSegTerms) {
@@ -641,6 +651,7 @@ __device__ double exact_seq_sum(const double* __restrict__ e, const double* __re
                 seg_terms(n, k0 + i * kSegTerms, lane, f, nx[d], fx);
                 if (i + kInFlight * kSumWaves < m) seg_load(e, n, k0 + (i + kInFlight * kSumWaves) * kSegTerms, lane, nx[d]);
                 if (i >= m) continue;
+                if (P) seg_store(p, n, k0 + i * kSegTerms, lane, fx);
                 const int ks = __builtin_amdgcn_readfirstlane(sh.grid[i]);
                 if (ks != kNoGrid) {
                     grid_count(fx, ks, i, lane, sh);
@@ -665,84 +676,84 @@ __device__ double exact_seq_sum(const double* __restrict__ e, const double* __re
     return s;
 }
 
+// Phase 3, Cdf::from_probs (coder.rs:43-81) from the two sums: extra[i] =
+// (u64)(p[i] * inv * rem + 0.5) and freq[i] = 1 + extra[i]; the surplus or deficit goes to
+// the last of the largest frequencies; then the cumulative frequencies.  The row's workgroup
+// gathers each chunk's used sum and its largest (frequency, last index) right after the sums, a
+// wave a chunk, 3b writes the chunk's cumulative frequencies from those.  Both read the f32
+// probabilities that the second sum left where the cumulative frequencies go, half of e's
+// bytes: k_cdf_freq_write 18.7 -> 15.0 us at 128 rows of 50,280, and the gathering, a kernel
+// of its own before (12 us and a launch), adds 7 us to the sums.  Every combination here is an integer sum
+// or a max, exact in any order.
+struct FreqRow {
+    double inv, rem;
+    uint64_t remaining;
+};
+__device__ __forceinline__ FreqRow freq_row(double sum_p, uint32_t n) {
+    FreqRow f;
+    f.remaining = (uint64_t)kCdfTotal - n;
+    f.inv = sum_p > 0.0 ? 1.0 / sum_p : 0.0;
+    f.rem = (double)f.remaining;
+    return f;
+}
+// (u64)(p inv rem + 0.5), truncated, NaN -> 0.  The sum of the probabilities is no smaller
+// than any of them (non-negative terms, monotone rounding), so this is 2^24 at most.
+__device__ __forceinline__ uint32_t extra_of(uint32_t p, const FreqRow& f) {
+    const double v = (double)__uint_as_float(p) * f.inv * f.rem + 0.5;
+    return v > 0.0 ? (uint32_t)v : 0u;
+}
+
+// Chunk c's used sum and largest frequency (one wave).
+__device__ void freq_part(const uint32_t* __restrict__ p, uint32_t n, uint32_t c, int lane, const FreqRow& f,
+                          ChunkPart& part) {
+    uint32_t mine = 0, most = 0, at = 0;   // (kChunk / 64 shares a lane: below 2^31)
+    const uint32_t c0 = c * kChunk, c1 = min(n, c0 + kChunk);
+    uint32_t v[kSpan];
+#pragma unroll
+    for (uint32_t j = 0; j < kSpan; j++) v[j] = p[min(c0 + 64 * j + (uint32_t)lane, n - 1)];
+    for (uint32_t k = c0; k < c1; k += 64 * kSpan) {
+        uint32_t nx[kSpan];
+#pragma unroll
+        for (uint32_t j = 0; j < kSpan; j++) nx[j] = p[min(k + 64 * (kSpan + j) + (uint32_t)lane, n - 1)];
+#pragma unroll
+        for (uint32_t j = 0; j < kSpan; j++) {
+            const uint32_t i = k + 64 * j + (uint32_t)lane;
+            const uint32_t x = i < c1 ? extra_of(v[j], f) : 0u;
+            mine += x;
+            const bool last = i < c1 && x >= most;   // the last of equal ones
+            most = last ? x : most;
+            at = last ? i : at;
+            v[j] = nx[j];
+        }
+    }
+    uint64_t used = mine, best = (uint64_t)(1u + most) << 32 | at;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        used += __shfl_xor(used, o);
+        const uint64_t b = __shfl_xor(best, o);
+        best = b > best ? b : best;
+    }
+    if (lane == 0) {
+        part.used = used;
+        part.best = best;
+    }
+}
+
 __global__ __launch_bounds__(kSumBlock) void k_cdf_sums(CdfArgs a) {
     __shared__ SumShared sh;
     const uint32_t row = blockIdx.x, n = a.n;
     const double* e = a.e + (size_t)row * n;
     const double* seg = a.seg + (size_t)row * segments(n);
-    const double s = exact_seq_sum(e, seg, n, 0.0, 1.0, [](double v) { return v; }, sh);
+    const double s = exact_seq_sum<false>(e, seg, n, 0.0, 1.0, [](double v) { return v; }, nullptr, sh);
     const double inv_sum = 1.0 / s;
-    const double sp = exact_seq_sum(e, seg, n, -0.0, inv_sum,
-                                    [inv_sum](double v) { return (double)prob_of(v, inv_sum); }, sh);
-    if (threadIdx.x == 0) {
-        a.sums[2 * row] = s;
-        a.sums[2 * row + 1] = sp;
-    }
-}
-
-// Phase 3, Cdf::from_probs (coder.rs:43-81) from the two sums: extra[i] =
-// (u64)(p[i] * inv * rem + 0.5) and freq[i] = 1 + extra[i]; the surplus or deficit goes to
-// the last of the largest frequencies; then the cumulative frequencies.  3a gathers each
-// chunk's used sum, its largest (frequency, last index) and its frequency total; 3b writes
-// the chunk's cumulative frequencies from those.  Every combination here is an integer sum
-// or a max, exact in any order.
-struct FreqRow {
-    double inv_sum, inv, rem;
-    uint64_t remaining;
-};
-__device__ __forceinline__ FreqRow freq_row(const CdfArgs& a, uint32_t row) {
-    FreqRow f;
-    const double s = a.sums[2 * row], sum_p = a.sums[2 * row + 1];
-    f.inv_sum = 1.0 / s;
-    f.remaining = (uint64_t)kCdfTotal - a.n;
-    f.inv = sum_p > 0.0 ? 1.0 / sum_p : 0.0;
-    f.rem = (double)f.remaining;
-    return f;
-}
-__device__ __forceinline__ uint64_t extra_of(double e, const FreqRow& f) {
-    return sat_u64((double)prob_of(e, f.inv_sum) * f.inv * f.rem + 0.5);
-}
-
-__global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_parts(CdfArgs a) {
-    __shared__ uint64_t sh64[kCdfBlock / 64];
-    __shared__ uint32_t sh32[kCdfBlock / 64];
-    const uint32_t c = blockIdx.x, row = blockIdx.y, n = a.n;
-    const FreqRow f = freq_row(a, row);
-    const double* e = a.e + (size_t)row * n;
-    uint64_t used = 0, best = 0;
-    uint32_t total = 0;
-    auto take = [&](double v, uint32_t i) {
-        const uint64_t x = extra_of(v, f);
-        const uint32_t fr = 1u + (uint32_t)x;
-        used += x;
-        total += fr;
-        const uint64_t key = ((uint64_t)fr << 32) | i;
-        best = key > best ? key : best;
-    };
-    const uint32_t i0 = c * kChunk, i1 = min(n, (c + 1) * kChunk);
-    if (((uintptr_t)e & 15) == 0) {
-        // two consecutive elements a lane (chunks start at even positions)
-        for (uint32_t i = i0 + 2 * threadIdx.x; i < i1; i += 2 * kCdfBlock) {
-            if (i + 2 <= i1) {
-                const double2 v = *(const double2*)(e + i);
-                take(v.x, i);
-                take(v.y, i + 1);
-            } else {
-                take(e[i], i);
-            }
-        }
-    } else {
-        for (uint32_t i = i0 + threadIdx.x; i < i1; i += kCdfBlock) take(e[i], i);
-    }
-    used = block_reduce<uint64_t>(used, [](uint64_t x, uint64_t y) { return x + y; }, sh64);
-    best = block_reduce<uint64_t>(best, [](uint64_t x, uint64_t y) { return x > y ? x : y; }, sh64);
-    total = block_reduce<uint32_t>(total, [](uint32_t x, uint32_t y) { return x + y; }, sh32);
-    if (threadIdx.x == 0) {
-        ChunkPart& p = a.part[(size_t)row * a.chunks + c];
-        p.used = used;
-        p.best = best;
-        p.total = total;
-    }
+    const double sp = exact_seq_sum<true>(e, seg, n, -0.0, inv_sum,
+                                          [inv_sum](double v) { return (double)prob_of(v, inv_sum); },
+                                          a.cdf + (size_t)row * (n + 1) + 1, sh);
+    if (threadIdx.x == 0) a.sums[row] = sp;
+    // (the probabilities were stored before the barriers of the sum)
+    const FreqRow f = freq_row(sp, n);
+    for (uint32_t c = uni(threadIdx.x / 64); c < a.chunks; c += kSumWaves)
+        freq_part(a.cdf + (size_t)row * (n + 1) + 1, n, c, threadIdx.x % 64, f, a.part[(size_t)row * a.chunks + c]);
 }
 
 // LDS index of a chunk position: one pad word per 32, so that both the coalesced pass
@@ -754,28 +765,31 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_write(CdfArgs a) {
     __shared__ uint32_t sh[kCdfBlock / 64];
     __shared__ uint32_t lfq[kChunk + kChunk / 32];   // the chunk's frequencies, then its cumulative ones
     const uint32_t c = blockIdx.x, row = blockIdx.y, n = a.n;
-    const FreqRow f = freq_row(a, row);
+    const FreqRow f = freq_row(a.sums[row], n);
     const ChunkPart* pr = a.part + (size_t)row * a.chunks;
     uint64_t used = 0, best = 0;
     uint32_t offset = 0;
     for (uint32_t i = 0; i < a.chunks; i++) {
         used += pr[i].used;
         best = pr[i].best > best ? pr[i].best : best;
-        if (i < c) offset += pr[i].total;
+        if (i < c) offset += (uint32_t)pr[i].used + kChunk;   // each frequency is 1 and its share (u32, wrapping)
     }
     const int64_t diff = (int64_t)f.remaining - (int64_t)used;
     const uint32_t at = (uint32_t)best;
     const uint32_t c0 = c * kChunk;
     if (diff != 0 && at < c0) offset = (uint32_t)((int64_t)offset + diff);   // u32 wrap, as the host's sum
-    const double* e = a.e + (size_t)row * n;
     uint32_t* cdf = a.cdf + (size_t)row * (n + 1);
-    // the chunk's frequencies, read coalesced (element c0 + t + 256 j)
+    // the chunk's frequencies, from the probabilities in the elements that its cumulative
+    // frequencies take at the end (read coalesced: element c0 + t + 256 j)
+    uint32_t prob[kSpan];
+#pragma unroll
+    for (uint32_t j = 0; j < kSpan; j++) prob[j] = cdf[1 + min(c0 + threadIdx.x + kCdfBlock * j, n - 1)];
 #pragma unroll
     for (uint32_t j = 0; j < kSpan; j++) {
         const uint32_t p = threadIdx.x + kCdfBlock * j, i = c0 + p;
         uint32_t v = 0;
         if (i < n) {
-            v = 1u + (uint32_t)extra_of(e[i], f);
+            v = 1u + extra_of(prob[j], f);
             if (diff != 0 && i == at) v = (uint32_t)((int64_t)v + diff);
         }
         lfq[pad_ix(p)] = v;
@@ -819,7 +833,7 @@ uint32_t cdf_chunks(uint32_t n) { return (n + kChunk - 1) / kChunk; }
 }  // namespace
 
 size_t cdf_scratch_bytes(uint32_t rows, uint32_t n) {
-    return (size_t)rows * n * 8 + (size_t)rows * 16 + (size_t)rows * segments(n) * 8 +
+    return (size_t)rows * n * 8 + (size_t)rows * 8 + (size_t)rows * segments(n) * 8 +
            (size_t)rows * cdf_chunks(n) * sizeof(ChunkPart);
 }
 
@@ -828,14 +842,13 @@ hipError_t cdf_launch(const float* logits, uint32_t rows, uint32_t n, void* scra
     const uint32_t chunks = cdf_chunks(n);
     double* e = (double*)scratch;
     double* sums = e + (size_t)rows * n;
-    double* seg = sums + 2 * (size_t)rows;
+    double* seg = sums + rows;
     ChunkPart* part = (ChunkPart*)(seg + (size_t)rows * segments(n));
     CdfArgs a{logits, rows, n, chunks, e, sums, seg, part, cdf};
     const dim3 grid(chunks, rows);
     k_cdf_max<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_exp<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_sums<<<dim3(rows), dim3(kSumBlock), 0, st>>>(a);
-    k_cdf_freq_parts<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_freq_write<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     return hipGetLastError();
 }
