@@ -521,10 +521,14 @@ int load_rwkv(const std::string& path, uint32_t profile) {
         ok = ok && rd.ok && make_rowmat(e, t.data(), (int)rows, (int)cols, 0);
     };
     // A LoRA stage: tiled for the matrix cores, or laid out for the exact kernels of the
-    // W8A8 and reference-order tiers.
+    // reference-order tier (whole 32-column blocks) or of the W8A8 tier.
+    bool blocks32 = true;
+    for (uint32_t r : R.lora) blocks32 = blocks32 && r % 32 == 0 && r <= (uint32_t)kMaxCols;
     auto lora = [&](RLayer& L, int k, bool first, size_t rows, size_t cols) {
         std::vector<float> t = rd.read(rows * cols);
-        if (G.r_a8 || G.r_exact)
+        if (G.r_exact && (first || blocks32))
+            ok = ok && rd.ok && make_rowmat(first ? L.e_x1[k] : L.e_x2[k], t.data(), (int)rows, (int)cols, 0);
+        else if (G.r_a8 || G.r_exact)
             ok = ok && rd.ok && make_lmat(first ? L.x1[k] : L.x2[k], t.data(), (int)rows, (int)cols);
         else ok = ok && rd.ok && make_tmat(first ? L.l1[k] : L.l2[k], t.data(), (int)rows, (int)cols, 0);
     };

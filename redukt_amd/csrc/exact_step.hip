@@ -30,6 +30,7 @@
 #include "mfma_common.h"
 #include "model.h"
 #include "portable_math.h"
+#include "rwkv_common.h"
 #include "step.h"
 
 #pragma clang fp contract(off)
@@ -143,7 +144,7 @@ __global__ __launch_bounds__(kEBlock) void k_norm_e(NormEArgs a) {
 
 // ---------------------------------------------------------------- projections
 
-enum : int { kEpiPlain = EXACT_STORE, kEpiIn = 1, kEpiRes = EXACT_RESID, kEpiRelu2 = EXACT_RELU2 };
+enum : int { kEpiPlain = EXACT_STORE, kEpiIn = 1, kEpiRes = EXACT_RESID, kEpiRelu2 = EXACT_RELU2, kEpiAct = 4 };
 
 struct GemvEArgs {
     RowMat w;               // [rows][cols]
@@ -163,11 +164,21 @@ struct GemvEArgs {
     int di;
     uint32_t chunks;        // chunks of 4 C streams
     int stride;             // LDS row stride of the staged activations
-    // Products 1 and 2 of a launch of three of one shape (grid y; product 0 is w, act,
-    // out): rows w_more[z - 1], input rows act_more[z - 1], outputs from out + out_more[z - 1].
-    RowMat w_more[2];
-    const float* act_more[2];
-    uint32_t out_more[2];
+};
+
+// One of the products of k_gemv_multi: out[b * ostride + r] = act of row r times stream b's
+// input row at x + b * ldx; its workgroups from blk0 on.
+struct GemvProduct {
+    RowMat w;
+    const float* x;
+    float* out;
+    uint32_t ldx, ostride, blk0;
+    int act, stride;
+};
+struct GemvMultiArgs {
+    GemvEArgs base;   // n and chunks
+    int count;
+    GemvProduct prod[kExactProducts];
 };
 
 // acc + w * x in the contract's arithmetic.
@@ -280,6 +291,7 @@ __device__ __forceinline__ void tile_decode(const TileRaw<Q8, R>& r, float (&w)[
 
 constexpr int kEWaves = kEBlock / kWave;
 constexpr int kEAhead = 8;        // 32-column blocks of weights in flight per wave
+constexpr int kEAheadShort = 4;   // the same where no row of a launch of several products is longer
 
 // One wave computes 8 R rows x 4 C streams.  Lane 8 l + r holds the reference's accumulators
 // l of row r of each octet, one register per stream: each step of a 32-column block adds one
@@ -302,15 +314,12 @@ constexpr int kEAhead = 8;        // 32-column blocks of weights in flight per w
 //
 // (Two workgroups a CU at least: at most 256 registers, so the products land in vector
 // registers, not in accumulation registers that the adds would have to be copied from.)
-template <bool Q8, bool FMA, int R, int C, int S, int EPI, int GB>
-__global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
+template <bool Q8, bool FMA, int R, int C, int S, int EPI, int GB, int AHEAD>
+__device__ __forceinline__ void gemv_e_body(const GemvEArgs& a, const RowMat& m, const float* act, uint32_t ldx, float* out,
+                                            uint32_t ostride, int stride, int actv, uint32_t lin) {
     extern __shared__ __align__(16) float acts[];   // [4 C][stride]
-    const uint32_t z = blockIdx.y;
-    const RowMat& m = z == 0 ? a.w : z == 1 ? a.w_more[0] : a.w_more[1];
-    const float* const act = z == 0 ? a.act : z == 1 ? a.act_more[0] : a.act_more[1];
-    float* const out = z == 0 ? a.out : a.out + (z == 1 ? a.out_more[0] : a.out_more[1]);
     const int parts = m.tiles() * (2 / R);   // tiles (R = 2) or their halves of 8 rows
-    const XcdTile job = xcd_tile(blockIdx.x, a.chunks, (uint32_t)((parts + kEWaves - 1) / kEWaves));
+    const XcdTile job = xcd_tile(lin, a.chunks, (uint32_t)((parts + kEWaves - 1) / kEWaves));
     if (!job.live) return;
     const int lane = threadIdx.x % kWave, wave = wave_index();
     const int cols = m.cols, nb = cols / 32;
@@ -325,9 +334,9 @@ __global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
     constexpr int kGB = GB > 0 ? GB : 1;   // (no division by zero in the other instantiation)
     const int ng = GB > 0 ? nb / kGB : 1;
     const float* scales = Q8 ? m.scales + (size_t)t * ng * kRowTile + r16 : nullptr;
-    TileRaw<Q8, R> raw[kEAhead];
+    TileRaw<Q8, R> raw[AHEAD];
 #pragma unroll
-    for (int i = 0; i < kEAhead; i++) raw[i] = tile_load<Q8, R, GB>(m, w0, min(i, nb - 1), half, lane, scales);
+    for (int i = 0; i < AHEAD; i++) raw[i] = tile_load<Q8, R, GB>(m, w0, min(i, nb - 1), half, lane, scales);
     const float sc_row = Q8 && GB == 0 ? scales[0] : 0.0f;
     // the epilogue's operands, requested with the products'
     float old[C], cs[C][3], cb = 0.0f;
@@ -337,7 +346,7 @@ __global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
 #pragma unroll
     for (int q = 0; q < C; q++) {
         const uint32_t b = b0 + 4 * q + (uint32_t)lane / 16;
-        old[q] = EPI == kEpiRes && row_live && b < a.n ? out[(size_t)b * a.ostride + r] : 0.0f;
+        old[q] = EPI == kEpiRes && row_live && b < a.n ? out[(size_t)b * ostride + r] : 0.0f;
         cs[q][0] = cs[q][1] = cs[q][2] = 0.0f;
         cst[q] = 0;
         if (conv && b < a.n) {
@@ -350,11 +359,10 @@ __global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
         cw = *(const float4*)(a.conv_w + (size_t)r * 4);
         cb = a.conv_b[r];
     }
-    const int stride = a.stride;
 #pragma unroll
     for (int s = 0; s < C; s++) {
         const int sr = wave + kEWaves * s;   // the wave's streams; S == 1: only the first is read
-        const float* src = act + (size_t)min(b0 + (uint32_t)sr, a.n - 1) * cols;
+        const float* src = act + (size_t)min(b0 + (uint32_t)sr, a.n - 1) * ldx;
         if (S == 4 || sr < S) {
 #pragma unroll 3
             for (int q = lane; q < cols / 4; q += kWave) {
@@ -405,17 +413,17 @@ __global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
 #pragma unroll
         for (int q = 0; q < C; q++) x[q] = xn[q];
     };
-    const int nbm = nb / kEAhead * kEAhead;
-    for (int k0 = 0; k0 < nbm; k0 += kEAhead) {
+    const int nbm = nb / AHEAD * AHEAD;
+    for (int k0 = 0; k0 < nbm; k0 += AHEAD) {
 #pragma unroll
-        for (int i = 0; i < kEAhead; i++) {
+        for (int i = 0; i < AHEAD; i++) {
             block(raw[i], k0 + i);
-            raw[i] = tile_load<Q8, R, GB>(m, w0, min(k0 + kEAhead + i, nb - 1), half, lane, scales);
+            raw[i] = tile_load<Q8, R, GB>(m, w0, min(k0 + AHEAD + i, nb - 1), half, lane, scales);
         }
     }
-    // the last nb % kEAhead blocks, already in raw[0 ..]
+    // the last nb % AHEAD blocks, already in raw[0 ..]
 #pragma unroll
-    for (int i = 0; i < kEAhead - 1; i++)
+    for (int i = 0; i < AHEAD - 1; i++)
         if (nbm + i < nb) block(raw[i], nbm + i);
     if (GB == 0) finish(sc_row);
     if (!row_live) return;
@@ -424,15 +432,17 @@ __global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
         const uint32_t b = b0 + 4 * q + (uint32_t)lane / 16;
         if (b >= a.n) continue;
         const float y = res[q];
-        if (EPI == kEpiPlain) {
-            out[(size_t)b * a.ostride + r] = y;
+        if (EPI == kEpiAct) {
+            out[(size_t)b * ostride + r] = activate(actv, y, r, m.rows);
+        } else if (EPI == kEpiPlain) {
+            out[(size_t)b * ostride + r] = y;
         } else if (EPI == kEpiRes) {
             // x += W_out * gated (model.rs:714-719): the residual add after the projection
-            out[(size_t)b * a.ostride + r] = old[q] + y;
+            out[(size_t)b * ostride + r] = old[q] + y;
         } else if (EPI == kEpiRelu2) {
             // squared_relu_into (tensor.rs:1386-1388): max(y, 0)^2, a NaN to 0
             const float v = y > 0.0f ? y : 0.0f;
-            out[(size_t)b * a.ostride + r] = v * v;
+            out[(size_t)b * ostride + r] = v * v;
         } else if (r >= a.di) {
             a.z[(size_t)b * a.di + (r - a.di)] = y;
         } else {
@@ -452,6 +462,26 @@ __global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
             a.u[(size_t)b * a.di + r] = val * lane_sigmoid_f(val);
         }
     }
+}
+
+template <bool Q8, bool FMA, int R, int C, int S, int EPI, int GB>
+__global__ __launch_bounds__(kEBlock, 2) void k_gemv_e(GemvEArgs a) {
+    gemv_e_body<Q8, FMA, R, C, S, EPI, GB, kEAhead>(a, a.w, a.act, (uint32_t)a.w.cols, a.out, a.ostride, a.stride, ACT_NONE,
+                                           blockIdx.x);
+}
+
+// Several F32 contract-1 products that do not read each other's outputs in one launch: RWKV-7's
+// receptance, key, value and first LoRA stages, then its second LoRA stages.  The LoRAs had a
+// kernel of their own, a lane per accumulator and every operand from memory: at 64 streams
+// 9.4 us a launch twice a layer beside 11.3 for the other three products; now 16.2 and 5.1.
+template <int R, int C, int S, int AHEAD>
+__global__ __launch_bounds__(kEBlock, 2) void k_gemv_multi(GemvMultiArgs a) {
+    int i = 0;
+    for (int k = 1; k < a.count; k++)
+        if (blockIdx.x >= a.prod[k].blk0) i = k;
+    const GemvProduct& p = a.prod[i];
+    gemv_e_body<false, false, R, C, S, kEpiAct, 0, AHEAD>(a.base, p.w, p.x, p.ldx, p.out, p.ostride, p.stride, p.act,
+                                                   blockIdx.x - p.blk0);
 }
 
 template <int R, int C, int S, int EPI>
@@ -487,24 +517,25 @@ int acts_stride(int cols, int quads) {
 // of 64 contract 2 at 32): in_proj 19.6, 19.7, 19.6, 20.1, 25.3 and 8.0, 8.7, 8.1, 8.7, 13.2;
 // x_proj 6.9, 10.9, 10.0, 16.4 and 5.2, 7.0, 6.8, 8.6; out_proj 12.0, 13.8, 14.4, 17.0 and 7.2,
 // 9.4, 8.8, 12.0; the head 229, 191, 218, 187, 200 and 67.6, 55.4, 55.6, 51.5, 53.7.
-Share exact_share(const RowMat& w, uint32_t products, uint32_t n) {
-    const uint64_t waves = (uint64_t)w.tiles() * 2 * products * ((n + 3) / 4);
+Share exact_share(uint32_t tiles, int cols, uint32_t n) {
+    const uint64_t waves = (uint64_t)tiles * 2 * ((n + 3) / 4);
     if (waves <= 10 * 1024) return Share{1, 1};
-    return Share{2, 32u * (uint32_t)w.cols <= kELdsMax ? 2 : 1};
+    return Share{2, 32u * (uint32_t)cols <= kELdsMax ? 2 : 1};
 }
 
-Launch gemv_e_launch(GemvPick pick, bool fma, int cls, const RowMat& w, const float* act, uint32_t n, GemvEArgs a,
-                     uint32_t products = 1) {
-    const Share s = exact_share(w, products, n);
+uint32_t gemv_e_grid(const RowMat& w, Share s, uint32_t chunks) {
+    return xcd_grid(chunks, (uint32_t)((w.tiles() * (2 / s.r) + kEWaves - 1) / kEWaves));
+}
+
+Launch gemv_e_launch(GemvPick pick, bool fma, int cls, const RowMat& w, const float* act, uint32_t n, GemvEArgs a) {
+    const Share s = exact_share((uint32_t)w.tiles(), w.cols, n);
     a.w = w;
     a.act = act;
     a.n = n;
     a.chunks = (n + 4 * s.c - 1) / (4 * s.c);
     a.stride = acts_stride(w.cols, s.c);
     const uint32_t lds = 16u * (uint32_t)s.c * (uint32_t)a.stride;
-    const uint32_t units = (uint32_t)((w.tiles() * (2 / s.r) + kEWaves - 1) / kEWaves);
-    return Launch::make(pick(n, s, w, fma), dim3(xcd_grid(a.chunks, units), products), dim3(kEBlock), lds,
-                        (uint32_t)cls, a);
+    return Launch::make(pick(n, s, w, fma), dim3(gemv_e_grid(w, s, a.chunks)), dim3(kEBlock), lds, (uint32_t)cls, a);
 }
 
 }  // namespace
@@ -520,17 +551,36 @@ Launch exact_gemv_launch(const RowMat& w, const float* act, uint32_t n, float* o
     return gemv_e_launch(pick, false, (int)cls, w, act, n, a);
 }
 
-Launch exact_gemv3_launch(const RowMat* const (&w)[3], const float* const (&act)[3], uint32_t n, float* out,
-                          const uint32_t (&out_off)[3], uint32_t ostride, uint32_t cls) {
-    GemvEArgs a{};
-    a.out = out + out_off[0];
-    a.ostride = ostride;
-    for (int k = 0; k < 2; k++) {
-        a.w_more[k] = *w[k + 1];
-        a.act_more[k] = act[k + 1];
-        a.out_more[k] = out_off[k + 1] - out_off[0];
+namespace {
+template <int AHEAD>
+const void* gemv_multi_fn(uint32_t n, Share s) {
+    if (s.r == 1) return n == 1 ? (const void*)k_gemv_multi<1, 1, 1, AHEAD> : (const void*)k_gemv_multi<1, 1, 4, AHEAD>;
+    return (const void*)k_gemv_multi<2, 2, 4, AHEAD>;   // (rows of at most 1,024 columns: s.c = 2)
+}
+}  // namespace
+
+Launch exact_gemv_multi_launch(const ExactProduct* prod, int count, uint32_t n, uint32_t cls) {
+    uint32_t tiles = 0;
+    int cols = 0;
+    for (int k = 0; k < count; k++) {
+        tiles += (uint32_t)prod[k].w->tiles();
+        cols = std::max(cols, prod[k].w->cols);
     }
-    return gemv_e_launch(gemv_e_pick<kEpiPlain>, false, (int)cls, *w[0], act[0], n, a, 3);
+    const Share s = exact_share(tiles, cols, n);
+    GemvMultiArgs a{};
+    a.base.n = n;
+    a.base.chunks = (n + 4 * s.c - 1) / (4 * s.c);
+    a.count = count;
+    uint32_t grid = 0, lds = 0;
+    for (int k = 0; k < count; k++) {
+        const ExactProduct& p = prod[k];
+        const int stride = acts_stride(p.w->cols, s.c);
+        a.prod[k] = GemvProduct{*p.w, p.x, p.out, p.ldx, p.ostride, grid, p.act, stride};
+        grid += gemv_e_grid(*p.w, s, a.base.chunks);
+        lds = std::max(lds, 16u * (uint32_t)s.c * (uint32_t)stride);
+    }
+    const void* fn = cols <= 32 * kEAheadShort ? gemv_multi_fn<kEAheadShort>(n, s) : gemv_multi_fn<kEAhead>(n, s);
+    return Launch::make(fn, dim3(grid), dim3(kEBlock), lds, cls, a);
 }
 
 void ExactStep::build(Pool& p, const StepIO& io, std::vector<Launch>& out, int& io_i, int& head_i, int& sm_i) const {

@@ -244,7 +244,10 @@ struct RLayer {
     TMat l1[4];                       // first LoRA stages [rank][d] (F32): w1, a1, g1, v1
     TMat l2[4];                       // second LoRA stages [d][rank] (F32): w2, a2, g2, v2
     TMat fk, fv;                      // [d_ffn][d], [d][d_ffn]
-    LMat x1[4], x2[4];                // the LoRA stages of the W8A8 and reference-order tiers (l1/l2 stay empty there)
+    // The LoRA stages of the W8A8 tier; of the reference-order tier in e_x1 and e_x2 (x2
+    // instead where a rank is not a multiple of 32, or above 1,024).  l1 and l2 stay empty there.
+    LMat x1[4], x2[4];
+    RowMat e_x1[4], e_x2[4];
     RowMat e_r, e_k, e_v, e_o, e_fk, e_fv;   // the reference-order tier's projections (the TMats stay empty there)
 };
 
@@ -392,10 +395,18 @@ struct ExactStep final : StepSource {
 enum ExactEpi : int { EXACT_STORE = 0, EXACT_RESID = 2, EXACT_RELU2 = 3 };
 Launch exact_gemv_launch(const RowMat& w, const float* act, uint32_t n, float* out, uint32_t ostride, int epi,
                          uint32_t cls);
-// Three such products of one shape in one launch (EXACT_STORE), product k's outputs from
-// out + out_off[k] (out_off ascending).
-Launch exact_gemv3_launch(const RowMat* const (&w)[3], const float* const (&act)[3], uint32_t n, float* out,
-                          const uint32_t (&out_off)[3], uint32_t ostride, uint32_t cls);
+// Up to kExactProducts such products of at most 1,024 columns, none reading another's output, in one launch: product
+// k's input rows are x + b * ldx, its outputs take the activation act (rwkv_common.h).
+constexpr int kExactProducts = 7;
+struct ExactProduct {
+    const RowMat* w;
+    const float* x;
+    uint32_t ldx;
+    float* out;
+    uint32_t ostride;
+    int act;
+};
+Launch exact_gemv_multi_launch(const ExactProduct* prod, int count, uint32_t n, uint32_t cls);
 
 struct RwkvStep final : StepSource {
     RwkvView m;

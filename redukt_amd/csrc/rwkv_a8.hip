@@ -31,8 +31,8 @@
 //
 // The reference-order tier (F32 weights, profile bit 6) runs the same element-wise kernels
 // with every projection an F32 GEMV in the reference's dot_avx2_order (mat_vec_mul_into,
-// tensor.rs:1602-1693; exact_gemv_launch, eight lanes per output; receptance, key and value
-// in one launch): k_shift_a8 hands all six
+// tensor.rs:1602-1693; exact_gemv_launch, eight lanes per output; receptance, key, value and
+// the first LoRA stages in one launch, the second ones in another): k_shift_a8 hands all six
 // token-shift inputs over as f32, and the receptance, key, value, output, FFN and head
 // products replace the int8 ones (the FFN key's squared ReLU in its epilogue), so the
 // logits are the CPU path's F32 logits bit for bit.
@@ -943,21 +943,30 @@ void RwkvStep::build_ref(Pool& p, const StepIO& io, std::vector<Launch>& out, in
         s1.outf[4] = mixf[kLoraA];
         s1.outf[5] = mixf[kLoraG];
         out.push_back(Launch::make(shift_a8_fn(6), dim3(n), dim3(kBlock), 0, KC_SHIFT, s1));
-        // receptance, key and value in one launch
-        const RowMat* const rkv_w[3] = {&L.e_r, &L.e_k, &L.e_v};
-        const float* const rkv_in[3] = {xr, xk, mixf[kLoraV]};
-        const uint32_t rkv_off[3] = {0u, (uint32_t)d, 2u * d};
-        out.push_back(exact_gemv3_launch(rkv_w, rkv_in, n, p.rkv, rkv_off, 3u * d, KC_PROJ));
-        ProjA8Builder p1(n, 0);
-        p1.lora(L.x1[kLoraW], mixf[kLoraW], d, ACT_TANH, lh[kLoraW], lsum);
-        p1.lora(L.x1[kLoraA], mixf[kLoraA], d, ACT_NONE, lh[kLoraA], lsum);
-        p1.lora(L.x1[kLoraG], mixf[kLoraG], d, ACT_SIGMOID, lh[kLoraG], lsum);
-        if (l != 0) p1.lora(L.x1[kLoraV], mixf[kLoraV], d, ACT_NONE, lh[kLoraV], lsum);
-        out.push_back(p1.launch());
-        ProjA8Builder p2(n, 0);
-        for (int k = 0; k < 4; k++)
-            if (k != kLoraV || l != 0) p2.lora(L.x2[k], lh[k], lsum, ACT_NONE, p.lorad + k * d, 4 * d);
-        out.push_back(p2.launch());
+        // receptance, key, value and the first LoRA stages in one launch
+        const uint32_t du = (uint32_t)d, lu = (uint32_t)lsum;
+        const ExactProduct first[kExactProducts] = {
+            {&L.e_r, xr, du, p.rkv, 3 * du, ACT_NONE},
+            {&L.e_k, xk, du, p.rkv + d, 3 * du, ACT_NONE},
+            {&L.e_v, mixf[kLoraV], du, p.rkv + 2 * d, 3 * du, ACT_NONE},
+            {&L.e_x1[kLoraW], mixf[kLoraW], du, lh[kLoraW], lu, ACT_TANH},
+            {&L.e_x1[kLoraA], mixf[kLoraA], du, lh[kLoraA], lu, ACT_NONE},
+            {&L.e_x1[kLoraG], mixf[kLoraG], du, lh[kLoraG], lu, ACT_SIGMOID},
+            {&L.e_x1[kLoraV], mixf[kLoraV], du, lh[kLoraV], lu, ACT_NONE},   // from layer 1 on
+        };
+        out.push_back(exact_gemv_multi_launch(first, l != 0 ? 7 : 6, n, KC_PROJ));
+        // second LoRA stages
+        if (L.e_x2[kLoraW].w != nullptr) {
+            ExactProduct second[4];
+            for (int k = 0; k < 4; k++) second[k] = {&L.e_x2[k], lh[k], lu, p.lorad + k * d, 4 * du, ACT_NONE};
+            static_assert(kLoraV == 3, "the value mix's stage last: from layer 1 on");
+            out.push_back(exact_gemv_multi_launch(second, l != 0 ? 4 : 3, n, KC_PROJ));
+        } else {
+            ProjA8Builder p2(n, 0);
+            for (int k = 0; k < 4; k++)
+                if (k != kLoraV || l != 0) p2.lora(L.x2[k], lh[k], lsum, ACT_NONE, p.lorad + k * d, 4 * d);
+            out.push_back(p2.launch());
+        }
         // the gated vector in f32 rows of d (its per-head maxima are not used here)
         WkvA8Args wa{p.rkv, p.lorad, L.w0, L.a0, L.v0, L.k_k, L.k_a, L.r_k, L.ln_x_w, L.ln_x_b,
                      p.wkv + l * wkv_layer, (size_t)D.nl * wkv_layer, p.vfirst, p.slots, p.scap, p.gatedf, d, p.pmax,

@@ -126,6 +126,23 @@ def test_bit_exact_rwkv7_0_1b(models, tier):
         orc.close()
 
 
+@pytest.mark.parametrize("ranks", [(32, 96, 160, 64), (128, 32, 32, 256), (40, 64, 64, 64)])
+@pytest.mark.parametrize("n", [1, 2, 5, 33, 560])
+def test_bit_exact_products_of_one_launch(tmp_path, ranks, n):
+    """Receptance, key, value and the LoRA stages share launches: one stream (its own kernel),
+    ragged chunks of four, rows of one to eight blocks of 32 beside each other, a rank that
+    is no multiple of 32 (the second stages' other kernel), and enough streams for 16 rows x
+    8 streams a wave."""
+    w, a, v, g = ranks
+    path = str(tmp_path / "m.rbin")
+    rwkv.write_synthetic(path, dataclasses.replace(SMALL, lora_w=w, lora_a=a, lora_v=v, lora_g=g), seed=sum(ranks))
+    with ffi.PluginBackend(path, profile=REF) as be:
+        orc = O.RwkvOracle(path, 0, cap=n)
+        be.batch_init(n)
+        run_equal(be, orc, n, 3, lambda s, t: (s * 41 + t * 73 + 5) % be.vocab, states=(0, n - 1))
+        orc.close()
+
+
 def test_batch_sizes_and_v1(models, tier):
     """One stream's bits do not depend on the batch it runs in, its position or its slot,
     and the v1 single-stream entry point gives the same bits."""
