@@ -1173,7 +1173,7 @@ __device__ __forceinline__ void scan_body(const ScanArgs& a, uint32_t sy, uint32
     // SPT streams per thread (streams SPT y .. SPT y + SPT - 1 of channel j): the channel's
     // operands (exp(A_log), the dt_proj row, biases, D) are loaded and decoded once for all
     // of them.  Every stream's arithmetic is the same whatever SPT is.
-    constexpr int kParts = (DR && NXB) ? 3 : 1;  // threads per x_proj output (fixed shape)
+    constexpr int kParts = (DR && NXB % 3 == 0 && NXB) ? 3 : 1;  // threads per x_proj output (fixed shape)
     constexpr int kDr = DR ? DR : kMaxDr;
     constexpr int kNxb = NXB ? NXB : kMaxNxb;
     const int di = a.di, dr = DR ? DR : a.dr, nxb = NXB ? NXB : a.nxb;
@@ -1418,6 +1418,13 @@ const void* scan_fn(bool q8dt, bool fast, int dr, int nxb, uint32_t spt) {
     }
     if (m130) return fast ? scan_fn_spt<false, true, 48, 48>(spt) : scan_fn_spt<false, false, 48, 48>(spt);
     return fast ? scan_fn_spt<false, true, 0, 0>(spt) : scan_fn_spt<false, false, 0, 0>(spt);
+}
+
+// The reference-order tier's, specialised for Mamba-130M's dt_rank in the same way: 48 fixed
+// terms of the dt_proj dot instead of 64 with a test each.
+template <bool Q8DT, bool FMA>
+const void* scan_exact_fn(bool m130) {
+    return m130 ? (const void*)k_scan<Q8DT, false, 48, 1, 1, FMA> : (const void*)k_scan<Q8DT, false, 0, 1, 1, FMA>;
 }
 
 // ---------------------------------------------------------------- k_mix_out
@@ -2466,9 +2473,9 @@ Launch scan_exact_launch(const DLayer& L, const Dims& D, Pool& p, uint32_t n, bo
     const int di = (int)D.di;
     ScanArgs sa = scan_args(L, D, p, n, nullptr, g32, ssm_layer);
     sa.nxb = 1;   // one block: each stream's complete x_proj outputs
-    const bool q8 = L.dt_q != nullptr;
-    const void* fs = q8 ? (fma ? (const void*)k_scan<true, false, 0, 1, 1, true> : (const void*)k_scan<true, false, 0, 1, 1, false>)
-                        : (fma ? (const void*)k_scan<false, false, 0, 1, 1, true> : (const void*)k_scan<false, false, 0, 1, 1, false>);
+    const bool q8 = L.dt_q != nullptr, m130 = D.dr == 48;
+    const void* fs = q8 ? (fma ? scan_exact_fn<true, true>(m130) : scan_exact_fn<true, false>(m130))
+                        : (fma ? scan_exact_fn<false, true>(m130) : scan_exact_fn<false, false>(m130));
     return Launch::make(fs, dim3(xcd_grid((di + kBlock - 1) / kBlock, n)), dim3(kBlock), 0, KC_SCAN, sa);
 }
 

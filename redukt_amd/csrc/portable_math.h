@@ -41,6 +41,30 @@ RDK_HD float round_even(float x) {
 // exp(x): clamp to [-87.34, 88.38], n = round_even(x*log2e), two-constant Cody-Waite
 // reduction, degree-5 polynomial, scale by 2^n built in the exponent field
 // (tensor.rs:765-794).
+#if defined(__HIP_DEVICE_COMPILE__)
+// On the device in 24 vector instructions instead of 37, with the same bits for every one of the
+// 2^32 inputs (compared): a NaN takes the lower bound (the lane rule below), the rounding is one
+// v_rndne (it may give -0 for +0, which leaves the result), and the scale one v_ldexp (one
+// rounding, as the multiplication by 2^n).  The reference-order scan, 18 of them a thread: 32
+// streams 6.9 -> 5.6 us, 100 streams 10.8 -> 10.0 (with its dt_rank fixed); the softmax of 128
+// rows of 50,280 22.5 -> 20.8.
+RDK_HD float exp_clamped_f(float x) {
+    x = x > -87.3365447505531f ? x : -87.3365447505531f;
+    x = __builtin_amdgcn_fmed3f(x, -87.3365447505531f, 88.3762626647949f);
+    const float n_f = __builtin_rintf(x * 1.44269504088896341f);
+    const float r = (x - n_f * 6.93145751953125E-1f) - n_f * 1.42860682030941723212E-6f;
+    const float r2 = r * r;
+    float p = 1.9875691500E-4f;
+    p = p * r + 1.3981999507E-3f;
+    p = p * r + 8.3334519073E-3f;
+    p = p * r + 4.1665795894E-2f;
+    p = p * r + 1.6666665459E-1f;
+    p = p * r + 5.0000001201E-1f;
+    p = (p * r2 + r) + 1.0f;
+    return __builtin_amdgcn_ldexpf(p, (int32_t)n_f);
+}
+RDK_HD float exp_f(float x) { return x != x ? x + x : exp_clamped_f(x); }
+#else
 RDK_HD float exp_f(float x) {
     const float lo = -87.3365447505531f, hi = 88.3762626647949f;
     x = x < lo ? lo : (x > hi ? hi : x);
@@ -57,12 +81,17 @@ RDK_HD float exp_f(float x) {
     p = (p * r2 + r) + 1.0f;
     return p * bits_to_f((uint32_t)(n + 127) << 23);
 }
+#endif
 
 // exp as one SIMD lane of the reference computes it: NaN becomes the lower clamp
 // (tensor.rs:877-879).  lane_exp_arg is that argument rule alone, for callers that pick
 // between the lane and the scalar form before one exp_f.
 RDK_HD float lane_exp_arg(float x) { return x != x ? -87.3365447505531f : x; }
+#if defined(__HIP_DEVICE_COMPILE__)
+RDK_HD float lane_exp_f(float x) { return exp_clamped_f(x); }
+#else
 RDK_HD float lane_exp_f(float x) { return exp_f(lane_exp_arg(x)); }
+#endif
 
 // 1 / (1 + exp(0 - x)) (tensor.rs:883-885).
 RDK_HD float lane_sigmoid_f(float x) { return 1.0f / (1.0f + lane_exp_f(0.0f - x)); }
