@@ -598,6 +598,12 @@ void dev_free_all() {
 // two chunks 47.6K / 77.5K; eight threads slicing every chunk, two chunks 55.2K / 97.5K,
 // four chunks 53.0K / 101.2K.
 constexpr size_t kOutChunkTarget = (size_t)4 << 20;
+// Logits of up to this many bytes are written by the head straight into pinned host memory: no
+// DMA behind the step (8 us each, in two chunks) and no copy threads, but the head's own stores
+// cross the bus, at about 17 GB/s.  us a call, with the DMAs / direct (Mamba-130M int8 through
+// the C ABI): 1 stream 420 / 376, 2 427 / 391, 4 430 / 411, 8 449 / 470, 32 578 / 854; RWKV-7
+// int8 1 stream 547 / 507, 4 (1 MB) 569 / 574; the reference-order tier 1 stream 738 / 698.
+constexpr size_t kDirectOutBytes = (size_t)900 << 10;
 constexpr size_t kOutMaxChunks = 4;
 constexpr size_t kOutRoundBytes = (size_t)32 << 20;
 constexpr unsigned kCopyThreadsMax = 8;   // the caller's thread and at most seven helpers
@@ -780,8 +786,7 @@ bool pool_alloc_rwkv(Pool& p, uint32_t cap) {
     p.gcap = (cap + 15) / 16;
     bool ok = pool_carve(p, [&](Carve& c) {
         c.take(p.slots, slot_words(cap));
-        c.take(p.d_slots, 3 * n);  // a step's n slots, its n tokens, then a word per stream for the CDF readers (one H2D copy)
-        for (Pool::Queued& q : p.queued) c.take(q.d_in, 3 * n);
+        c.take(p.d_slots, n);
         c.take(p.x, n * d);
         c.take(p.vfirst, n * d);
         c.take(p.rkv, n * 3 * d);
@@ -824,8 +829,7 @@ bool pool_alloc(Pool& p, uint32_t cap) {
     const size_t ns = p.scap;
     bool ok = pool_carve(p, [&](Carve& c) {
         c.take(p.slots, slot_words(cap));
-        c.take(p.d_slots, 3 * n);  // a step's n slots, its n tokens, then a word per stream for the CDF readers (one H2D copy)
-        for (Pool::Queued& q : p.queued) c.take(q.d_in, 3 * n);
+        c.take(p.d_slots, n);
         c.take(p.x, n * d);
         c.take(p.xw, xw_elems(D, cap));
         c.take(p.ssp, ssp_floats(D, cap));
@@ -942,21 +946,29 @@ bool copy_out(Pool& p, void* dst, const void* src, size_t bytes) {
 }
 
 // pool_forward semantics (mamba_cuda.cu:604-635): validate on the host (nothing is
-// launched on INVALID_ARGUMENT), stage slots/tokens through pinned memory, enqueue the
-// step, copy the n rows back to the caller (through pinned staging, chunked) and wait.
+// launched on INVALID_ARGUMENT), put slots and tokens into pinned memory, enqueue the step,
+// which reads them there, copy the n rows back to the caller (through pinned staging,
+// chunked) and wait.
 int pool_forward(Pool& p, uint32_t n, const uint32_t* slots, const uint32_t* tokens, float* out, bool probs) {
     memset(p.seen, 0, p.cap);
     for (uint32_t b = 0; b < n; b++) {
         if (slots[b] >= p.cap || p.seen[slots[b]] || tokens[b] >= G.dims.vocab) return BACKEND_INVALID_ARGUMENT;
         p.seen[slots[b]] = 1;
     }
-    // the n slots, then the n tokens, in one staging run and one copy
     memcpy(p.h_slots, slots, sizeof(uint32_t) * n);
     memcpy(p.h_slots + n, tokens, sizeof(uint32_t) * n);
-    if (hipMemcpyAsync(p.d_slots, p.h_slots, sizeof(uint32_t) * 2 * n, hipMemcpyHostToDevice, G.stream) != hipSuccess)
-        return BACKEND_FORWARD_FAILED;
-    if (run_step(p, n, p.d_slots, p.d_slots + n, p.out, probs, false) != hipSuccess) return BACKEND_FORWARD_FAILED;
-    if (!copy_out(p, out, p.out, sizeof(float) * n * G.dims.vocab)) return BACKEND_FORWARD_FAILED;
+    // (the embedding reads the two lists over the bus once: an H2D copy before the step took
+    // 8 to 13 us a call)
+    const size_t bytes = sizeof(float) * n * vocab_of_model();
+    if (!probs && bytes <= kDirectOutBytes && bytes <= p.out_stage_bytes) {
+        if (run_step(p, n, p.h_slots, p.h_slots + n, (float*)p.h_out, false, false) != hipSuccess ||
+            hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0]))
+            return BACKEND_FORWARD_FAILED;
+        memcpy(out, p.h_out, bytes);
+        return BACKEND_OK;
+    }
+    if (run_step(p, n, p.h_slots, p.h_slots + n, p.out, probs, false) != hipSuccess) return BACKEND_FORWARD_FAILED;
+    if (!copy_out(p, out, p.out, bytes)) return BACKEND_FORWARD_FAILED;
     return BACKEND_OK;
 }
 
@@ -1289,11 +1301,10 @@ int32_t redukt_backend_forward_batch_probs(uint32_t n_streams, const uint32_t* s
 // The CDF kernels' scratch (exp values and the two sums per row) and, for the host-buffer
 // entry point, the CDF rows themselves: one allocation, grown on demand (the stream is
 // synchronized before the old one is freed).
-bool cdf_space(uint32_t rows, uint32_t n, bool with_out, void** scratch, uint32_t** out, uint32_t** pick = nullptr) {
+bool cdf_space(uint32_t rows, uint32_t n, bool with_out, void** scratch, uint32_t** out) {
     const size_t sb = (cdf_scratch_bytes(rows, n) + 255) & ~(size_t)255;
     const size_t ob = with_out ? ((size_t)rows * (n + 1) * 4 + 255) & ~(size_t)255 : 0;
-    // pick: the coder's three or four values per row
-    const size_t need = sb + ob + (pick ? (size_t)rows * 4 * 4 : 0);
+    const size_t need = sb + ob;
     if (need > G.cdf_bytes) {
         if (G.cdf_mem) {
             if (hipStreamSynchronize(G.stream) != hipSuccess) return false;
@@ -1309,7 +1320,6 @@ bool cdf_space(uint32_t rows, uint32_t n, bool with_out, void** scratch, uint32_
     }
     *scratch = G.cdf_mem;
     if (out) *out = (uint32_t*)((unsigned char*)G.cdf_mem + sb);
-    if (pick) *pick = (uint32_t*)((unsigned char*)G.cdf_mem + sb + ob);
     return true;
 }
 
@@ -1331,10 +1341,7 @@ int32_t redukt_backend_forward_batch_cdf(uint32_t n_streams, const uint32_t* slo
     if (!cdf_space(n_streams, V, true, &scratch, &d_cdf)) return BACKEND_FORWARD_FAILED;
     memcpy(p.h_slots, slots, sizeof(uint32_t) * n_streams);
     memcpy(p.h_slots + n_streams, tokens, sizeof(uint32_t) * n_streams);
-    if (hipMemcpyAsync(p.d_slots, p.h_slots, sizeof(uint32_t) * 2 * n_streams, hipMemcpyHostToDevice, G.stream) !=
-        hipSuccess)
-        return BACKEND_FORWARD_FAILED;
-    if (run_step(p, n_streams, p.d_slots, p.d_slots + n_streams, p.out, false, false) != hipSuccess ||
+    if (run_step(p, n_streams, p.h_slots, p.h_slots + n_streams, p.out, false, false) != hipSuccess ||
         cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) != hipSuccess)
         return BACKEND_FORWARD_FAILED;
     if (!copy_out(p, out_cdf, d_cdf, sizeof(uint32_t) * n_streams * (size_t)(V + 1))) return BACKEND_FORWARD_FAILED;
@@ -1342,10 +1349,10 @@ int32_t redukt_backend_forward_batch_cdf(uint32_t n_streams, const uint32_t* slo
 }
 
 namespace {
-// forward_batch_cdf_sym and _find: one H2D copy of the slots, the tokens and each stream's
-// next symbol (sym) or decoder target (find) through the pool's pinned staging; the step,
-// the device CDF and the kernel that reads the rows; `per` u32 a stream back through the
-// pinned output staging, waited for by polling its event.
+// forward_batch_cdf_sym and _find: the slots, the tokens and each stream's next symbol (sym)
+// or decoder target (find) in the pool's pinned memory; the step, the device CDF and the
+// kernel that reads the rows and writes `per` u32 a stream into the pinned output staging,
+// waited for by polling an event.
 int32_t forward_batch_cdf_read(uint32_t n_streams, const uint32_t* slots, const uint32_t* tokens,
                                const uint32_t* third, uint32_t* out, uint32_t vocab_size, bool find) {
     if (!G.ready || G.batch.cap == 0) return BACKEND_INIT_FAILED;
@@ -1364,23 +1371,19 @@ int32_t forward_batch_cdf_read(uint32_t n_streams, const uint32_t* slots, const 
     const size_t out_bytes = sizeof(uint32_t) * per * n_streams;
     if (out_bytes > p.out_stage_bytes) return BACKEND_FORWARD_FAILED;   // staging holds >= 4 u32 a stream
     void* scratch = nullptr;
-    uint32_t *d_cdf = nullptr, *d_out = nullptr;
-    if (!cdf_space(n_streams, V, true, &scratch, &d_cdf, &d_out)) return BACKEND_FORWARD_FAILED;
+    uint32_t* d_cdf = nullptr;
+    if (!cdf_space(n_streams, V, true, &scratch, &d_cdf)) return BACKEND_FORWARD_FAILED;
     memcpy(p.h_slots, slots, sizeof(uint32_t) * n_streams);
     memcpy(p.h_slots + n_streams, tokens, sizeof(uint32_t) * n_streams);
     memcpy(p.h_slots + 2 * n_streams, third, sizeof(uint32_t) * n_streams);
-    if (hipMemcpyAsync(p.d_slots, p.h_slots, sizeof(uint32_t) * 3 * n_streams, hipMemcpyHostToDevice, G.stream) !=
-        hipSuccess)
-        return BACKEND_FORWARD_FAILED;
-    const uint32_t* d_third = p.d_slots + 2 * n_streams;
-    if (run_step(p, n_streams, p.d_slots, p.d_slots + n_streams, p.out, false, false) != hipSuccess ||
+    const uint32_t* h_third = p.h_slots + 2 * n_streams;
+    uint32_t* const h_res = (uint32_t*)p.h_out;
+    if (run_step(p, n_streams, p.h_slots, p.h_slots + n_streams, p.out, false, false) != hipSuccess ||
         cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) != hipSuccess ||
-        (find ? cdf_find_launch(d_cdf, n_streams, V, d_third, d_out, G.stream)
-              : cdf_pick_launch(d_cdf, n_streams, V, d_third, d_out, G.stream)) != hipSuccess)
+        (find ? cdf_find_launch(d_cdf, n_streams, V, h_third, h_res, G.stream)
+              : cdf_pick_launch(d_cdf, n_streams, V, h_third, h_res, G.stream)) != hipSuccess)
         return BACKEND_FORWARD_FAILED;
-    if (hipMemcpyAsync(p.h_out, d_out, out_bytes, hipMemcpyDeviceToHost, G.stream) != hipSuccess ||
-        hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0]))
-        return BACKEND_FORWARD_FAILED;
+    if (hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0])) return BACKEND_FORWARD_FAILED;
     memcpy(out, p.h_out, out_bytes);
     return BACKEND_OK;
 }
@@ -1416,20 +1419,16 @@ int32_t redukt_backend_forward_batch_cdf_sym_submit(uint32_t n_streams, const ui
     }
     if (n_streams > 0) {
         void* scratch = nullptr;
-        uint32_t *d_cdf = nullptr, *d_pick = nullptr;
+        uint32_t* d_cdf = nullptr;
         // (a regrown scratch synchronizes the stream first, the other call's work included)
-        if (!cdf_space(n_streams, V, true, &scratch, &d_cdf, &d_pick)) return BACKEND_FORWARD_FAILED;
+        if (!cdf_space(n_streams, V, true, &scratch, &d_cdf)) return BACKEND_FORWARD_FAILED;
         memcpy(q->h_in, slots, sizeof(uint32_t) * n_streams);
         memcpy(q->h_in + n_streams, tokens, sizeof(uint32_t) * n_streams);
         memcpy(q->h_in + 2 * n_streams, next_syms, sizeof(uint32_t) * n_streams);
         const bool ok =
-            hipMemcpyAsync(q->d_in, q->h_in, sizeof(uint32_t) * 3 * n_streams, hipMemcpyHostToDevice, G.stream) ==
-                hipSuccess &&
-            run_step(p, n_streams, q->d_in, q->d_in + n_streams, p.out, false, false) == hipSuccess &&
+            run_step(p, n_streams, q->h_in, q->h_in + n_streams, p.out, false, false) == hipSuccess &&
             cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) == hipSuccess &&
-            cdf_pick_launch(d_cdf, n_streams, V, q->d_in + 2 * n_streams, d_pick, G.stream) == hipSuccess &&
-            hipMemcpyAsync(q->h_res, d_pick, sizeof(uint32_t) * 3 * n_streams, hipMemcpyDeviceToHost, G.stream) ==
-                hipSuccess;
+            cdf_pick_launch(d_cdf, n_streams, V, q->h_in + 2 * n_streams, q->h_res, G.stream) == hipSuccess;
         if (!ok) {
             // what was queued finishes before its buffers can be reused
             (void)hipStreamSynchronize(G.stream);

@@ -171,9 +171,10 @@ struct Pool {
     float* pmax = nullptr;       // [rows16][heads] each head's largest magnitude in gatedf
     float* out = nullptr;        // [cap][vocab] logits or probabilities
     uint32_t* slots = nullptr;   // [cap] slots of the current step (validated copy)
-    uint32_t* d_slots = nullptr; // [3 cap] H2D target of the synchronous entry points: n slots, n tokens,
-                                 // then n next symbols or decoder targets (the CDF readers)
-    uint32_t* h_slots = nullptr; // [3 cap] pinned staging of the same
+    uint32_t* d_slots = nullptr; // [cap] H2D target of a reset's slots
+    // [3 cap] pinned: the synchronous entry points' n slots, n tokens, then n next symbols or decoder targets (the
+    // CDF readers), read there by the step's kernels; a reset's slots
+    uint32_t* h_slots = nullptr;
     // Pinned staging of the outputs handed back to host memory (up to one round of
     // out_stage_bytes), with one completion event per chunk of a round (at most four).
     unsigned char* h_out = nullptr;
@@ -181,12 +182,11 @@ struct Pool {
     hipEvent_t out_ev[32] = {};
     uint8_t* seen = nullptr;     // host duplicate check, cap bytes
     // Queued calls (forward_batch_cdf_sym_submit / _wait): at most kQueued in flight, each
-    // with its own inputs (3 cap u32: slots, tokens, next symbols; pinned and on the
-    // device), its results (3 cap u32, pinned) and its completion event.
+    // with its own inputs (3 cap u32: slots, tokens, next symbols) and results (3 cap u32),
+    // both pinned, and its completion event.
     static constexpr uint32_t kQueued = 2;
     struct Queued {
         uint32_t* h_in = nullptr;
-        uint32_t* d_in = nullptr;
         uint32_t* h_res = nullptr;
         hipEvent_t done = nullptr;
         uint64_t ticket = 0;   // 0: free

@@ -510,3 +510,27 @@ def test_split_device_check_covers_every_part(models, monkeypatch):
         for (c0, x0), (c1, x1) in zip(s3_bad, state(3)):
             assert np.array_equal(c0, c1) and np.array_equal(x0, x1)
         assert np.array_equal(bits(bad[keep]), bits(good))
+
+
+@pytest.mark.parametrize("profile", [0, ffi.PROFILE_Q8_ROW | ffi.PROFILE_Q8_SMALL, ffi.PROFILE_Q8_ROW | ffi.PROFILE_GEMV,
+                                     ffi.PROFILE_Q8_G64 | ffi.PROFILE_EXACT])
+def test_host_logits_equal_device_logits(full_model, profile):
+    """The head writes few streams' logits straight into pinned host memory (up to 900 KB: four
+    streams of this vocabulary); more go through its own array and DMAs.  Both are the
+    device entry point's bits, with the two kinds of call in turn on one pool."""
+    with ffi.PluginBackend(full_model, profile=profile) as be:
+        be.batch_init(2 * 33)
+        for t in range(3):
+            for n in (1, 4, 5, 33, 2):
+                a, b = list(range(n)), list(range(33, 33 + n))     # the same tokens on two sets of slots
+                toks = np.arange(n, dtype=np.int32) * 131 + 7 * t + 1
+                host = np.empty((n, be.vocab), np.float32)
+                be.forward_batch(a, toks.tolist(), host)
+                bufs = [hip.DeviceBuffer.from_array(np.asarray(b, np.int32)), hip.DeviceBuffer.from_array(toks),
+                        hip.DeviceBuffer(n * be.vocab * 4)]
+                be.forward_batch_device(n, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr)
+                hip.stream_sync(be.stream())
+                dev = bufs[2].download(np.uint32, n * be.vocab).reshape(n, -1)
+                for x in bufs:
+                    x.close()
+                assert np.array_equal(host.view(np.uint32), dev), (t, n)
