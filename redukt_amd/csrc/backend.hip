@@ -1379,9 +1379,7 @@ int32_t forward_batch_cdf_read(uint32_t n_streams, const uint32_t* slots, const 
     const uint32_t* h_third = p.h_slots + 2 * n_streams;
     uint32_t* const h_res = (uint32_t*)p.h_out;
     if (run_step(p, n_streams, p.h_slots, p.h_slots + n_streams, p.out, false, false) != hipSuccess ||
-        cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) != hipSuccess ||
-        (find ? cdf_find_launch(d_cdf, n_streams, V, h_third, h_res, G.stream)
-              : cdf_pick_launch(d_cdf, n_streams, V, h_third, h_res, G.stream)) != hipSuccess)
+        cdf_read_launch(p.out, n_streams, V, scratch, d_cdf, find, h_third, h_res, G.stream) != hipSuccess)
         return BACKEND_FORWARD_FAILED;
     if (hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0])) return BACKEND_FORWARD_FAILED;
     memcpy(out, p.h_out, out_bytes);
@@ -1427,8 +1425,8 @@ int32_t redukt_backend_forward_batch_cdf_sym_submit(uint32_t n_streams, const ui
         memcpy(q->h_in + 2 * n_streams, next_syms, sizeof(uint32_t) * n_streams);
         const bool ok =
             run_step(p, n_streams, q->h_in, q->h_in + n_streams, p.out, false, false) == hipSuccess &&
-            cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) == hipSuccess &&
-            cdf_pick_launch(d_cdf, n_streams, V, q->h_in + 2 * n_streams, q->h_res, G.stream) == hipSuccess;
+            cdf_read_launch(p.out, n_streams, V, scratch, d_cdf, false, q->h_in + 2 * n_streams, q->h_res, G.stream) ==
+                hipSuccess;
         if (!ok) {
             // what was queued finishes before its buffers can be reused
             (void)hipStreamSynchronize(G.stream);

@@ -761,24 +761,48 @@ __global__ __launch_bounds__(kSumBlock) void k_cdf_sums(CdfArgs a) {
 // conflicts.
 __device__ __forceinline__ uint32_t pad_ix(uint32_t p) { return p + p / 32; }
 
-__global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_write(CdfArgs a) {
-    __shared__ uint32_t sh[kCdfBlock / 64];
-    __shared__ uint32_t lfq[kChunk + kChunk / 32];   // the chunk's frequencies, then its cumulative ones
-    const uint32_t c = blockIdx.x, row = blockIdx.y, n = a.n;
-    const FreqRow f = freq_row(a.sums[row], n);
+// What a row's chunks add up to, in every thread.
+struct RowFix {
+    FreqRow f;
+    int64_t diff;      // the fix-up
+    uint32_t at;       // the element that takes it
+    uint64_t most;     // that element's frequency before it
+    uint32_t total;    // cdf[n]
+};
+// Chunk c's first cumulative frequency (u32, wrapping, as the host's sum; each frequency is 1
+// and its share).
+__device__ __forceinline__ RowFix row_fix(const CdfArgs& a, uint32_t row) {
+    RowFix x;
+    x.f = freq_row(a.sums[row], a.n);
     const ChunkPart* pr = a.part + (size_t)row * a.chunks;
     uint64_t used = 0, best = 0;
-    uint32_t offset = 0;
     for (uint32_t i = 0; i < a.chunks; i++) {
         used += pr[i].used;
         best = pr[i].best > best ? pr[i].best : best;
-        if (i < c) offset += (uint32_t)pr[i].used + kChunk;   // each frequency is 1 and its share (u32, wrapping)
     }
-    const int64_t diff = (int64_t)f.remaining - (int64_t)used;
-    const uint32_t at = (uint32_t)best;
-    const uint32_t c0 = c * kChunk;
-    if (diff != 0 && at < c0) offset = (uint32_t)((int64_t)offset + diff);   // u32 wrap, as the host's sum
-    uint32_t* cdf = a.cdf + (size_t)row * (n + 1);
+    x.diff = (int64_t)x.f.remaining - (int64_t)used;
+    x.at = (uint32_t)best;
+    x.most = best >> 32;
+    x.total = (uint32_t)((int64_t)(a.n + used) + x.diff);
+    return x;
+}
+__device__ __forceinline__ uint32_t chunk_offset(const CdfArgs& a, uint32_t row, uint32_t c, const RowFix& x) {
+    const ChunkPart* pr = a.part + (size_t)row * a.chunks;
+    uint32_t offset = 0;
+    for (uint32_t i = 0; i < c; i++) offset += (uint32_t)pr[i].used + kChunk;
+    return x.at < c * kChunk ? (uint32_t)((int64_t)offset + x.diff) : offset;
+}
+
+struct ChunkShared {
+    uint32_t wave[kCdfBlock / 64];
+    uint32_t cum[kChunk + kChunk / 32];   // element c0 + r's cumulative frequency (its own included) at pad_ix(r)
+};
+// Chunk c's cumulative frequencies into sh.cum (every thread of the workgroup; it may be
+// called again once all have read).
+__device__ __forceinline__ void chunk_cum(const CdfArgs& a, uint32_t row, uint32_t c, const RowFix& x, uint32_t offset,
+                                          ChunkShared& sh) {
+    const uint32_t c0 = c * kChunk, n = a.n;
+    const uint32_t* cdf = a.cdf + (size_t)row * (n + 1);
     // the chunk's frequencies, from the probabilities in the elements that its cumulative
     // frequencies take at the end (read coalesced: element c0 + t + 256 j)
     uint32_t prob[kSpan];
@@ -789,10 +813,10 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_write(CdfArgs a) {
         const uint32_t p = threadIdx.x + kCdfBlock * j, i = c0 + p;
         uint32_t v = 0;
         if (i < n) {
-            v = 1u + extra_of(prob[j], f);
-            if (diff != 0 && i == at) v = (uint32_t)((int64_t)v + diff);
+            v = 1u + extra_of(prob[j], x.f);
+            if (i == x.at) v = (uint32_t)((int64_t)v + x.diff);
         }
-        lfq[pad_ix(p)] = v;
+        sh.cum[pad_ix(p)] = v;
     }
     __syncthreads();
     // thread t: kSpan consecutive elements; exclusive scan of the thread totals
@@ -800,7 +824,7 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_write(CdfArgs a) {
     uint32_t mine = 0;
 #pragma unroll
     for (uint32_t j = 0; j < kSpan; j++) {
-        fq[j] = lfq[pad_ix(threadIdx.x * kSpan + j)];
+        fq[j] = sh.cum[pad_ix(threadIdx.x * kSpan + j)];
         mine += fq[j];
     }
     const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
@@ -810,20 +834,112 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_write(CdfArgs a) {
         const uint32_t up = __shfl_up(incl, o);
         if (lane >= o) incl += up;
     }
-    if (lane == 63) sh[w] = incl;
+    if (lane == 63) sh.wave[w] = incl;
     __syncthreads();
     uint32_t cum = offset + incl - mine;
 #pragma unroll
     for (int i = 0; i < kCdfBlock / 64; i++)
-        if (i < w) cum += sh[i];
-    if (c == 0 && threadIdx.x == 0) cdf[0] = 0;
+        if (i < w) cum += sh.wave[i];
 #pragma unroll
     for (uint32_t j = 0; j < kSpan; j++) {
         cum += fq[j];
-        lfq[pad_ix(threadIdx.x * kSpan + j)] = cum;   // each thread rewrites only its own positions
+        sh.cum[pad_ix(threadIdx.x * kSpan + j)] = cum;   // each thread rewrites only its own positions
     }
     __syncthreads();
-    for (uint32_t r = threadIdx.x; r < kChunk && c0 + r < n; r += kCdfBlock) cdf[c0 + r + 1] = lfq[pad_ix(r)];
+}
+
+__global__ __launch_bounds__(kCdfBlock) void k_cdf_freq_write(CdfArgs a) {
+    __shared__ ChunkShared sh;
+    const uint32_t c = blockIdx.x, row = blockIdx.y, n = a.n, c0 = c * kChunk;
+    const RowFix x = row_fix(a, row);
+    chunk_cum(a, row, c, x, chunk_offset(a, row, c, x), sh);
+    uint32_t* cdf = a.cdf + (size_t)row * (n + 1);
+    if (c == 0 && threadIdx.x == 0) cdf[0] = 0;
+    for (uint32_t r = threadIdx.x; r < kChunk && c0 + r < n; r += kCdfBlock) cdf[c0 + r + 1] = sh.cum[pad_ix(r)];
+}
+
+// What the range coder reads of a row, straight from the shares: one workgroup a row works
+// out the one chunk it needs, so the rows' cumulative frequencies are not written (at 128 rows of
+// 50,280 k_cdf_freq_write's 15 us and 5 more for a kernel that reads three of them back; now 8, with the search 10).
+// FIND false: symbol key[r] is known (coder.rs:163-177 via encode_symbol): out[3r] = cdf[r][key],
+// out[3r + 1] = cdf[r][key + 1], out[3r + 2] = cdf[r][n], the total.  (The host checked it
+// against n; the clamp keeps every read inside the row whatever it holds.)
+// FIND true: the symbol s that the decoder's binary search finds for its target key[r]
+// (coder.rs:100-115): out[4r] = s, out[4r + 1] = cdf[r][s], out[4r + 2] = cdf[r][s + 1],
+// out[4r + 3] = cdf[r][n]; s = n (both bounds cdf[r][n]) where the target is not below the
+// total.  The frequencies are positive but for the one that takes a deficit of the shares.
+// Where it stays non-negative the row rises and the search finds the first element above the
+// target: first the chunk, then the element.  Else the search is done as it is, probe by probe.
+template <bool FIND>
+__global__ __launch_bounds__(kCdfBlock) void k_cdf_read(CdfArgs a, const uint32_t* __restrict__ key, uint32_t* __restrict__ out) {
+    __shared__ ChunkShared sh;
+    __shared__ uint32_t first;
+    const uint32_t row = blockIdx.x, n = a.n;
+    const RowFix x = row_fix(a, row);
+    const uint32_t k = key[row];
+    uint32_t s, chunk, offset;
+    if (!FIND) {
+        s = min(k, n - 1);
+        chunk = s / kChunk;
+        offset = chunk_offset(a, row, chunk, x);
+        chunk_cum(a, row, chunk, x, offset, sh);
+    } else if ((int64_t)x.most + x.diff >= 0) {
+        if (k >= x.total) {
+            if (threadIdx.x == 0) {
+                uint32_t* o = out + 4 * (size_t)row;
+                o[0] = n;
+                o[1] = o[2] = o[3] = x.total;
+            }
+            return;
+        }
+        uint32_t end = 0;   // of the chunk, before the fix-up
+        for (chunk = 0; chunk + 1 < a.chunks; chunk++) {
+            end += (uint32_t)a.part[(size_t)row * a.chunks + chunk].used + kChunk;
+            if ((x.at < (chunk + 1) * kChunk ? (uint32_t)((int64_t)end + x.diff) : end) > k) break;
+        }
+        offset = chunk_offset(a, row, chunk, x);
+        if (threadIdx.x == 0) first = kChunk;
+        chunk_cum(a, row, chunk, x, offset, sh);
+        uint32_t mine = kChunk;
+#pragma unroll
+        for (int j = (int)kSpan - 1; j >= 0; j--) {
+            const uint32_t r = threadIdx.x * kSpan + (uint32_t)j;
+            if (chunk * kChunk + r < n && sh.cum[pad_ix(r)] > k) mine = r;
+        }
+        if (mine < kChunk) atomicMin(&first, mine);
+        __syncthreads();
+        s = chunk * kChunk + first;
+    } else {
+        uint32_t lo = 0, hi = n;
+        chunk = 0xffffffffu;
+        offset = 0;
+        auto load = [&](uint32_t c) {
+            if (c == chunk) return;
+            __syncthreads();   // the chunk before has been read
+            chunk = c;
+            offset = chunk_offset(a, row, c, x);
+            chunk_cum(a, row, c, x, offset, sh);
+        };
+        while (lo < hi) {
+            const uint32_t m = lo + (hi - lo) / 2;
+            load(m / kChunk);
+            if (sh.cum[pad_ix(m % kChunk)] <= k)
+                lo = m + 1;
+            else
+                hi = m;
+        }
+        s = lo;
+        if (s < n) load(s / kChunk);
+    }
+    if (threadIdx.x != 0) return;
+    const uint32_t r = s % kChunk;
+    const uint32_t below = s == n ? x.total : r > 0 ? sh.cum[pad_ix(r - 1)] : offset;
+    const uint32_t above = s == n ? x.total : sh.cum[pad_ix(r)];
+    uint32_t* o = out + (FIND ? 4 : 3) * (size_t)row;
+    if (FIND) *o++ = s;
+    o[0] = below;
+    o[1] = above;
+    o[2] = x.total;
 }
 
 }  // namespace
@@ -837,106 +953,38 @@ size_t cdf_scratch_bytes(uint32_t rows, uint32_t n) {
            (size_t)rows * cdf_chunks(n) * sizeof(ChunkPart);
 }
 
-hipError_t cdf_launch(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* cdf, hipStream_t st) {
-    if (rows == 0) return hipSuccess;
+namespace {
+// The probabilities of every row (in the CDF elements) and the chunks' shares.
+CdfArgs cdf_shares(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* cdf, hipStream_t st) {
     const uint32_t chunks = cdf_chunks(n);
     double* e = (double*)scratch;
     double* sums = e + (size_t)rows * n;
     double* seg = sums + rows;
     ChunkPart* part = (ChunkPart*)(seg + (size_t)rows * segments(n));
-    CdfArgs a{logits, rows, n, chunks, e, sums, seg, part, cdf};
+    const CdfArgs a{logits, rows, n, chunks, e, sums, seg, part, cdf};
     const dim3 grid(chunks, rows);
     k_cdf_max<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_exp<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_sums<<<dim3(rows), dim3(kSumBlock), 0, st>>>(a);
-    k_cdf_freq_write<<<grid, dim3(kCdfBlock), 0, st>>>(a);
-    return hipGetLastError();
-}
-
-namespace {
-// What the range coder reads of row r when its next symbol is known (coder.rs:163-177 via
-// encode_symbol): out[3r] = cdf[r][sym[r]], out[3r + 1] = cdf[r][sym[r] + 1], out[3r + 2] =
-// cdf[r][n], the total.  The host checked sym[r] < n; the clamp keeps every read inside
-// the row whatever it holds.
-__global__ __launch_bounds__(256) void k_cdf_pick(const uint32_t* __restrict__ cdf, uint32_t rows, uint32_t n,
-                                                  const uint32_t* __restrict__ sym, uint32_t* __restrict__ out) {
-    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
-    if (r >= rows) return;
-    const uint32_t s = min(sym[r], n - 1);
-    const uint32_t* row = cdf + (size_t)r * (n + 1);
-    out[3 * (size_t)r] = row[s];
-    out[3 * (size_t)r + 1] = row[s + 1];
-    out[3 * (size_t)r + 2] = row[n];
+    return a;
 }
 }  // namespace
 
-hipError_t cdf_pick_launch(const uint32_t* cdf, uint32_t rows, uint32_t n, const uint32_t* sym, uint32_t* out,
-                           hipStream_t st) {
+hipError_t cdf_launch(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* cdf, hipStream_t st) {
     if (rows == 0) return hipSuccess;
-    k_cdf_pick<<<dim3((rows + 255) / 256), dim3(256), 0, st>>>(cdf, rows, n, sym, out);
+    const CdfArgs a = cdf_shares(logits, rows, n, scratch, cdf, st);
+    k_cdf_freq_write<<<dim3(a.chunks, rows), dim3(kCdfBlock), 0, st>>>(a);
     return hipGetLastError();
 }
 
-namespace {
-// The symbol the range decoder finds in row r for its target cum[r] (coder.rs:100-115, the
-// binary search of decode_symbol) with what it reads next: out[4r] = s, out[4r + 1] =
-// cdf[r][s], out[4r + 2] = cdf[r][s + 1], out[4r + 3] = cdf[r][n]; s = n (both bounds
-// cdf[r][n]) when cum[r] >= cdf[r][n].  One wave a row takes six levels of the search
-// per round trip to memory: lane k (1..63) is node k of those levels' tree in heap order
-// (children 2k: hi = mid, 2k + 1: lo = mid + 1), works out its node's interval from the
-// bits of k and evaluates the node's test; the wave then walks the tree from the ballot.
-// Every decision is the host search's own (the same mid of the same interval), so the
-// result equals it for any row contents, monotone or not.
-constexpr uint32_t kFindRows = 4;   // rows (waves) a workgroup
-
-__global__ __launch_bounds__(64 * kFindRows) void k_cdf_find(const uint32_t* __restrict__ cdf, uint32_t rows,
-                                                              uint32_t n, const uint32_t* __restrict__ cum,
-                                                              uint32_t* __restrict__ out) {
-    const uint32_t r = blockIdx.x * kFindRows + threadIdx.x / 64, lane = threadIdx.x % 64;
-    if (r >= rows) return;   // whole waves
-    const uint32_t* row = cdf + (size_t)r * (n + 1);
-    const uint32_t t = cum[r];
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        bool right = false;
-        if (lane > 0) {
-            uint32_t a = lo, b = hi;
-            for (int d = 30 - __clz(lane); d >= 0 && a < b; d--) {   // path bits below the leading one
-                const uint32_t m = a + (b - a) / 2;
-                if ((lane >> d) & 1)
-                    a = m + 1;
-                else
-                    b = m;
-            }
-            if (a < b) right = row[a + (b - a) / 2 + 1] <= t;
-        }
-        const uint64_t bits = __ballot(right);
-        for (uint32_t level = 0, node = 1; level < 6 && lo < hi; level++) {
-            const uint32_t m = lo + (hi - lo) / 2;
-            if ((bits >> node) & 1) {
-                lo = m + 1;
-                node = 2 * node + 1;
-            } else {
-                hi = m;
-                node = 2 * node;
-            }
-        }
-    }
-    if (lane == 0) {
-        const uint32_t total = row[n];
-        uint32_t* o = out + 4 * (size_t)r;
-        o[0] = lo;
-        o[1] = lo < n ? row[lo] : total;
-        o[2] = lo < n ? row[lo + 1] : total;
-        o[3] = total;
-    }
-}
-}  // namespace
-
-hipError_t cdf_find_launch(const uint32_t* cdf, uint32_t rows, uint32_t n, const uint32_t* cum, uint32_t* out,
-                           hipStream_t st) {
+hipError_t cdf_read_launch(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* space, bool find,
+                           const uint32_t* key, uint32_t* out, hipStream_t st) {
     if (rows == 0) return hipSuccess;
-    k_cdf_find<<<dim3((rows + kFindRows - 1) / kFindRows), dim3(64 * kFindRows), 0, st>>>(cdf, rows, n, cum, out);
+    const CdfArgs a = cdf_shares(logits, rows, n, scratch, space, st);
+    if (find)
+        k_cdf_read<true><<<dim3(rows), dim3(kCdfBlock), 0, st>>>(a, key, out);
+    else
+        k_cdf_read<false><<<dim3(rows), dim3(kCdfBlock), 0, st>>>(a, key, out);
     return hipGetLastError();
 }
 

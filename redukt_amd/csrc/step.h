@@ -66,13 +66,12 @@ bool gemv_cpl_supported(int cpl);
 // cdf_from_logits (cdf_step.hip); `scratch` holds cdf_scratch_bytes(rows, n).
 size_t cdf_scratch_bytes(uint32_t rows, uint32_t n);
 hipError_t cdf_launch(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* cdf, hipStream_t st);
-// out[3r .. 3r + 2] = cdf[r][sym[r]], cdf[r][sym[r] + 1], cdf[r][n] for rows r (cdf rows of n + 1).
-hipError_t cdf_pick_launch(const uint32_t* cdf, uint32_t rows, uint32_t n, const uint32_t* sym, uint32_t* out,
-                           hipStream_t st);
-// The decoder's symbol for each row's target cumulative frequency, with its two bounds and
-// the row's total (4 u32 a row).
-hipError_t cdf_find_launch(const uint32_t* cdf, uint32_t rows, uint32_t n, const uint32_t* cum, uint32_t* out,
-                           hipStream_t st);
+// What the range coder reads of each row, without the rows themselves (`space`: rows x (n + 1)
+// u32 of scratch).  !find: out[3r .. 3r + 2] = cdf[r][key[r]], cdf[r][key[r] + 1], cdf[r][n];
+// find: the decoder's symbol for the target key[r], its two bounds and the total (4 u32 a row).
+// key and out may be pinned host memory.
+hipError_t cdf_read_launch(const float* logits, uint32_t rows, uint32_t n, void* scratch, uint32_t* space, bool find,
+                           const uint32_t* key, uint32_t* out, hipStream_t st);
 
 namespace {
 

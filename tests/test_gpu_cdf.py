@@ -22,7 +22,7 @@ the CPU tests pin to the oracle and the reference's exp goldens:
 import numpy as np
 import pytest
 
-from redukt_amd import codec, ffi, hip, lockstep, rwkv, synth
+from redukt_amd import codec, ffi, hip, lockstep, rbin, rwkv, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -303,6 +303,44 @@ def test_forward_batch_cdf_rwkv7(tmp_path):
     with ffi.PluginBackend(p, profile=2) as be:
         be.batch_init(16)
         step_pair(be, 8, 2, seed=3)
+
+
+@pytest.mark.parametrize("scale,vocab", [(0.0, 50280), (0.0, 300), (0.0, 65536), (40.0, 4096), (40.0, 4097), (400.0, 8193),
+                                         (1.0, 2)])
+def test_readers_on_flat_and_peaked_rows(tmp_path, scale, vocab):
+    """The coder's readers work out one chunk of the row: rows of one chunk, of whole chunks and
+    one element more; all mass on few symbols; equal logits, whose rounded-up shares leave a
+    deficit larger than any frequency where the vocabulary is large (the last one wraps, so the
+    row falls at its end) and a surplus where it is small.  Targets sit on both sides of every
+    chunk's edges and of the fix-up's element."""
+    dims = rbin.MambaDims(vocab=vocab, d_model=64, n_layer=1)
+    w = dict(synth.mamba_tensors(dims, 3))
+    w["emb"] = (w["emb"] * scale).astype(np.float32)
+    p = str(tmp_path / "m.rbin")
+    rbin.write_rbin(p, dims, w.items())
+    n = 24
+    with ffi.PluginBackend(p, profile=0) as be:
+        be.batch_init(3 * n)
+        toks = [b * 31 % vocab for b in range(n)]
+        logits = np.empty((n, vocab), np.float32)
+        be.forward_batch(list(range(n)), toks, logits)
+        rows = [codec.cdf_from_logits(r) for r in logits]
+        edges = [0, 1, vocab // 2, vocab - 2, vocab - 1, 4095, 4096, 4097, 8191, 8192, int(np.argmax(np.diff(rows[0].astype(np.int64))))]
+        syms = np.array([edges[b % len(edges)] % vocab for b in range(n)], np.uint32)
+        got = np.empty(3 * n, np.uint32)
+        assert be.forward_batch_cdf_sym(list(range(n, 2 * n)), toks, syms, got) == ffi.BackendResult.OK
+        assert np.array_equal(got, np.array([v for b in range(n) for v in (rows[b][syms[b]], rows[b][syms[b] + 1], rows[b][vocab])]))
+        for off in (0, -1, 1):
+            be.batch_reset(list(range(2 * n, 3 * n)))
+            targets = np.array([(int(rows[b][syms[b]]) + off) % 2**32 for b in range(n)], np.uint32)
+            targets[:3] = [(1 << 24) - 1, 1 << 24, 2**32 - 1]
+            found = np.empty(4 * n, np.uint32)
+            assert be.forward_batch_cdf_find(list(range(2 * n, 3 * n)), toks, targets, found) == ffi.BackendResult.OK
+            want = []
+            for b in range(n):
+                k, t = codec.lookup(rows[b], int(targets[b])), rows[b][vocab]
+                want += [k, rows[b][k], rows[b][k + 1], t] if k < vocab else [vocab, t, t, t]
+            assert np.array_equal(found, np.array(want, np.uint32)), off
 
 
 def test_lockstep_device_cdf_bytes_equal_host_cdf(full_model, monkeypatch):
