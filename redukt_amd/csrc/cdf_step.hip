@@ -455,6 +455,9 @@ __device__ double exact_segment(double (&fx)[kTerms], double s, int lane) {
 #pragma unroll
             for (uint32_t j = 0; j < kTerms; j++) g[j].a += unit_step(w.step[j] | (w.lead[j] & first), g[j].d);
         }
+        const double incl = wave_incl_sum((g[0].a + g[1].a) + (g[2].a + g[3].a));
+        const double end = T0 + lane_f64(incl, 63);
+        if (__ballot(bad[0] || bad[1] || bad[2] || bad[3]) == 0 && end < top) return uni(ldexp(end, -ks));   // no event
         double c[kTerms];   // the lane's inclusive prefix
         double mine = 0.0;
 #pragma unroll
@@ -462,7 +465,6 @@ __device__ double exact_segment(double (&fx)[kTerms], double s, int lane) {
             mine += g[j].a;
             c[j] = mine;
         }
-        const double incl = wave_incl_sum(mine);
         const double base = T0 + dpp_f64<0x138>(incl);   // wave_shr:1 (lane 0 reads 0)
         // the lane's first term that is bad or takes T to the top of the binade
         bool hit = false;
@@ -476,8 +478,7 @@ __device__ double exact_segment(double (&fx)[kTerms], double s, int lane) {
             T_ev = h ? (j > 0 ? base + c[j - 1] : base) : T_ev;
             x_ev = h ? fx[j] : x_ev;
         }
-        const uint64_t has = __ballot(hit);
-        if (has == 0) return uni(ldexp(T0 + lane_f64(incl, 63), -ks));   // no event: T0 + total < top
+        const uint64_t has = __ballot(hit);   // some lane: T passes the top, or a term is bad
         const int src = (int)uni((uint32_t)__builtin_ctzll(has));
         s = uni(ldexp(lane_f64(T_ev, src), -ks) + lane_f64(x_ev, src));
         const uint32_t done = (uint32_t)src * kTerms + (uint32_t)__builtin_amdgcn_readlane((int)at, src);
