@@ -31,7 +31,7 @@
 //
 // The reference-order tier (F32 weights, profile bit 6) runs the same element-wise kernels
 // with every projection an F32 GEMV in the reference's dot_avx2_order (mat_vec_mul_into,
-// tensor.rs:1602-1693; exact_gemv_launch, eight lanes per output; receptance, key, value and
+// tensor.rs:1602-1693; exact_gemv_launch; receptance, key, value and
 // the first LoRA stages in one launch, the second ones in another): k_shift_a8 hands all six
 // token-shift inputs over as f32, and the receptance, key, value, output, FFN and head
 // products replace the int8 ones (the FFN key's squared ReLU in its epilogue), so the
