@@ -704,6 +704,19 @@ __device__ __forceinline__ uint32_t extra_of(uint32_t p, const FreqRow& f) {
     return v > 0.0 ? (uint32_t)v : 0u;
 }
 
+// A wave's used sum and largest (frequency, last index) from its lanes' sum, largest share and
+// that one's index.
+__device__ __forceinline__ void part_reduce(uint32_t mine, uint32_t most, uint32_t at, uint64_t& used, uint64_t& best) {
+    used = mine;
+    best = (uint64_t)(1u + most) << 32 | at;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        used += __shfl_xor(used, o);
+        const uint64_t b = __shfl_xor(best, o);
+        best = b > best ? b : best;
+    }
+}
+
 // Chunk c's used sum and largest frequency (one wave).
 __device__ void freq_part(const uint32_t* __restrict__ p, uint32_t n, uint32_t c, int lane, const FreqRow& f,
                           ChunkPart& part) {
@@ -727,16 +740,61 @@ __device__ void freq_part(const uint32_t* __restrict__ p, uint32_t n, uint32_t c
             v[j] = nx[j];
         }
     }
-    uint64_t used = mine, best = (uint64_t)(1u + most) << 32 | at;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        used += __shfl_xor(used, o);
-        const uint64_t b = __shfl_xor(best, o);
-        best = b > best ? b : best;
-    }
+    uint64_t used, best;
+    part_reduce(mine, most, at, used, best);
     if (lane == 0) {
         part.used = used;
         part.best = best;
+    }
+}
+
+// A row of one segment (a byte vocabulary): one wave adds its terms in order, both times from
+// the same registers, and takes their shares from there.  Bound by the two chains of adds and the
+// launches: the whole CDF of 128 / 512 rows of 256 takes 13.7 / 14.4 us, 19.5 for 128 rows through
+// k_cdf_sums; two segments gain from it no more (its second one would be another chain of 256).
+__global__ __launch_bounds__(64) void k_cdf_sums_short(CdfArgs a) {
+    __shared__ double terms[kSegTerms];
+    const uint32_t row = blockIdx.x, n = a.n;
+    const int lane = threadIdx.x;
+    double raw[kTerms], fx[kTerms];
+    seg_load(a.e + (size_t)row * n, n, 0, lane, raw);
+    auto sum = [&](double s) {
+#pragma unroll
+        for (uint32_t j = 0; j < kTerms; j++) terms[(uint32_t)lane * kTerms + j] = fx[j];
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // this wave's LDS stores done
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t t = 0; t < n; t += 16) {
+            double v[16];
+#pragma unroll
+            for (uint32_t k = 0; k < 16; k++) v[k] = terms[t + k];
+#pragma unroll
+            for (uint32_t k = 0; k < 16; k++) s += v[k];
+        }
+        __builtin_amdgcn_wave_barrier();
+        return uni(s);
+    };
+    seg_terms(n, 0, lane, [](double v) { return v; }, raw, fx);
+    const double inv_sum = 1.0 / sum(0.0);
+    seg_terms(n, 0, lane, [inv_sum](double v) { return (double)prob_of(v, inv_sum); }, raw, fx);
+    seg_store(a.cdf + (size_t)row * (n + 1) + 1, n, 0, lane, fx);
+    const double sp = sum(-0.0);
+    const FreqRow f = freq_row(sp, n);
+    uint32_t mine = 0, most = 0, at = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kTerms; j++) {
+        const uint32_t i = (uint32_t)lane * kTerms + j;
+        const uint32_t x = i < n ? extra_of(__float_as_uint((float)fx[j]), f) : 0u;
+        const bool last = i < n && x >= most;   // the last of equal ones
+        mine += x;
+        most = last ? x : most;
+        at = last ? i : at;
+    }
+    uint64_t used, best;
+    part_reduce(mine, most, at, used, best);
+    if (lane == 0) {
+        a.sums[row] = sp;
+        a.part[row].used = used;
+        a.part[row].best = best;
     }
 }
 
@@ -966,7 +1024,10 @@ CdfArgs cdf_shares(const float* logits, uint32_t rows, uint32_t n, void* scratch
     const dim3 grid(chunks, rows);
     k_cdf_max<<<grid, dim3(kCdfBlock), 0, st>>>(a);
     k_cdf_exp<<<grid, dim3(kCdfBlock), 0, st>>>(a);
-    k_cdf_sums<<<dim3(rows), dim3(kSumBlock), 0, st>>>(a);
+    if (n <= kSegTerms)
+        k_cdf_sums_short<<<dim3(rows), dim3(64), 0, st>>>(a);
+    else
+        k_cdf_sums<<<dim3(rows), dim3(kSumBlock), 0, st>>>(a);
     return a;
 }
 }  // namespace
