@@ -265,12 +265,12 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_exp(CdfArgs a) {
 // by term.  The running sum of these rows stays below 2^24 (each term <= 1, n < 2^24), so
 // the grid is always finer than 1.
 //
-// 128 rows of 50,280 normal logits of standard deviations 1 to 4: 57 us (67 with the shares
-// after the sums), where 4,096 terms of the whole workgroup a round in order (two barriers,
-// 1.7 us each, about 46 rounds a row) took 121; the whole CDF 175 -> 112.  Of a row, each sum: 1.8 us to classify, 7 to count (51 MB
-// of e over all rows at 7 TB/s; the second sum 8 to 17, by how many of its terms are ties), 10
-// to 14 in the chain, whose lone wave issues at a third of the vector rate: about 1.3 us for
-// each uncounted segment with the run before it.
+// Bound by latency.  128 rows of 50,280 normal logits of standard deviations 1 to 4: 57 us (67
+// with the shares after the sums), where 4,096 terms of the whole workgroup a round in order
+// (two barriers, 1.7 us each, about 46 rounds a row) took 121; the whole CDF 175 -> 112.  Of a
+// row, each sum: 1.8 us to classify, 7 to count (51 MB of e over all rows at 7 TB/s; the second
+// sum 8 to 17, by how many of its terms are ties), 10 to 14 in the chain, whose lone wave issues
+// at a third of the vector rate: about 1.3 us for each uncounted segment with the run before it.
 // The same value in every lane, made visibly uniform (scalar registers): the round loop's
 // control values come from LDS, and without this the compiler treats the loop as divergent
 // (exec masking, and copies of the prefetched terms that wait for their loads every round).

@@ -395,8 +395,9 @@ struct ExactStep final : StepSource {
 enum ExactEpi : int { EXACT_STORE = 0, EXACT_RESID = 2, EXACT_RELU2 = 3 };
 Launch exact_gemv_launch(const RowMat& w, const float* act, uint32_t n, float* out, uint32_t ostride, int epi,
                          uint32_t cls);
-// Up to kExactProducts such products of at most 1,024 columns, none reading another's output, in one launch: product
-// k's input rows are x + b * ldx, its outputs take the activation act (rwkv_common.h).
+// Up to kExactProducts such products of at most 1,024 columns, none reading another's output,
+// in one launch: product k's input rows are x + b * ldx, its outputs take the activation act
+// (rwkv_common.h).
 constexpr int kExactProducts = 7;
 struct ExactProduct {
     const RowMat* w;
