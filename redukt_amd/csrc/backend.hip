@@ -908,6 +908,15 @@ bool event_wait(hipEvent_t e) {
     }
 }
 
+// The end of a host call that failed after part of it may have been queued: waits for that part,
+// which still reads the pool's pinned inputs and writes its pinned outputs, so that the next call
+// can use them.
+int32_t forward_failed() {
+    G.runner.sync_parts();
+    (void)hipStreamSynchronize(G.stream);
+    return BACKEND_FORWARD_FAILED;
+}
+
 // The first `bytes` of the device array src into the caller's host buffer dst, through the
 // pool's pinned staging, a round at a time: all of a round's chunks are queued D2H (each
 // followed by its event) behind the step; the caller alone polls for the first chunk (which
@@ -963,12 +972,12 @@ int pool_forward(Pool& p, uint32_t n, const uint32_t* slots, const uint32_t* tok
     if (!probs && bytes <= kDirectOutBytes && bytes <= p.out_stage_bytes) {
         if (run_step(p, n, p.h_slots, p.h_slots + n, (float*)p.h_out, false, false) != hipSuccess ||
             hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0]))
-            return BACKEND_FORWARD_FAILED;
+            return forward_failed();
         memcpy(out, p.h_out, bytes);
         return BACKEND_OK;
     }
-    if (run_step(p, n, p.h_slots, p.h_slots + n, p.out, probs, false) != hipSuccess) return BACKEND_FORWARD_FAILED;
-    if (!copy_out(p, out, p.out, bytes)) return BACKEND_FORWARD_FAILED;
+    if (run_step(p, n, p.h_slots, p.h_slots + n, p.out, probs, false) != hipSuccess || !copy_out(p, out, p.out, bytes))
+        return forward_failed();
     return BACKEND_OK;
 }
 
@@ -979,15 +988,14 @@ int pool_reset(Pool& p, uint32_t n, const uint32_t* slots) {
         if (s >= p.cap) return BACKEND_INVALID_ARGUMENT;
     }
     if (n == 0) return BACKEND_OK;
-    // Every earlier call that used p.h_slots ended with a stream synchronize, so the
-    // staging buffer is free to overwrite.
+    // Every earlier call that used p.h_slots waited for what it had queued, also where it
+    // failed (forward_failed), so the staging buffer is free to overwrite.
     for (uint32_t b = 0; b < n; b++) p.h_slots[b] = slots ? slots[b] : b;
     if (hipMemcpyAsync(p.d_slots, p.h_slots, sizeof(uint32_t) * n, hipMemcpyHostToDevice, G.stream) != hipSuccess)
-        return BACKEND_FORWARD_FAILED;
+        return forward_failed();
     const hipError_t e = G.kind == kKindRwkv ? enqueue_reset_rwkv(G.rdims, p, p.d_slots, n, G.stream)
                                              : enqueue_reset(G.dims, p, p.d_slots, n, G.stream);
-    if (e != hipSuccess) return BACKEND_FORWARD_FAILED;
-    if (hipStreamSynchronize(G.stream) != hipSuccess) return BACKEND_FORWARD_FAILED;
+    if (e != hipSuccess || hipStreamSynchronize(G.stream) != hipSuccess) return forward_failed();
     return BACKEND_OK;
 }
 
@@ -1342,9 +1350,9 @@ int32_t redukt_backend_forward_batch_cdf(uint32_t n_streams, const uint32_t* slo
     memcpy(p.h_slots, slots, sizeof(uint32_t) * n_streams);
     memcpy(p.h_slots + n_streams, tokens, sizeof(uint32_t) * n_streams);
     if (run_step(p, n_streams, p.h_slots, p.h_slots + n_streams, p.out, false, false) != hipSuccess ||
-        cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) != hipSuccess)
-        return BACKEND_FORWARD_FAILED;
-    if (!copy_out(p, out_cdf, d_cdf, sizeof(uint32_t) * n_streams * (size_t)(V + 1))) return BACKEND_FORWARD_FAILED;
+        cdf_launch(p.out, n_streams, V, scratch, d_cdf, G.stream) != hipSuccess ||
+        !copy_out(p, out_cdf, d_cdf, sizeof(uint32_t) * n_streams * (size_t)(V + 1)))
+        return forward_failed();
     return BACKEND_OK;
 }
 
@@ -1379,9 +1387,9 @@ int32_t forward_batch_cdf_read(uint32_t n_streams, const uint32_t* slots, const 
     const uint32_t* h_third = p.h_slots + 2 * n_streams;
     uint32_t* const h_res = (uint32_t*)p.h_out;
     if (run_step(p, n_streams, p.h_slots, p.h_slots + n_streams, p.out, false, false) != hipSuccess ||
-        cdf_read_launch(p.out, n_streams, V, scratch, d_cdf, find, h_third, h_res, G.stream) != hipSuccess)
-        return BACKEND_FORWARD_FAILED;
-    if (hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0])) return BACKEND_FORWARD_FAILED;
+        cdf_read_launch(p.out, n_streams, V, scratch, d_cdf, find, h_third, h_res, G.stream) != hipSuccess ||
+        hipEventRecord(p.out_ev[0], G.stream) != hipSuccess || !event_wait(p.out_ev[0]))
+        return forward_failed();
     memcpy(out, p.h_out, out_bytes);
     return BACKEND_OK;
 }
@@ -1423,20 +1431,12 @@ int32_t redukt_backend_forward_batch_cdf_sym_submit(uint32_t n_streams, const ui
         memcpy(q->h_in, slots, sizeof(uint32_t) * n_streams);
         memcpy(q->h_in + n_streams, tokens, sizeof(uint32_t) * n_streams);
         memcpy(q->h_in + 2 * n_streams, next_syms, sizeof(uint32_t) * n_streams);
-        const bool ok =
-            run_step(p, n_streams, q->h_in, q->h_in + n_streams, p.out, false, false) == hipSuccess &&
-            cdf_read_launch(p.out, n_streams, V, scratch, d_cdf, false, q->h_in + 2 * n_streams, q->h_res, G.stream) ==
-                hipSuccess;
-        if (!ok) {
-            // what was queued finishes before its buffers can be reused
-            (void)hipStreamSynchronize(G.stream);
-            return BACKEND_FORWARD_FAILED;
-        }
+        if (run_step(p, n_streams, q->h_in, q->h_in + n_streams, p.out, false, false) != hipSuccess ||
+            cdf_read_launch(p.out, n_streams, V, scratch, d_cdf, false, q->h_in + 2 * n_streams, q->h_res, G.stream) !=
+                hipSuccess)
+            return forward_failed();
     }
-    if (hipEventRecord(q->done, G.stream) != hipSuccess) {
-        (void)hipStreamSynchronize(G.stream);
-        return BACKEND_FORWARD_FAILED;
-    }
+    if (hipEventRecord(q->done, G.stream) != hipSuccess) return forward_failed();
     q->n = n_streams;
     q->ticket = g_next_ticket++;
     *ticket = q->ticket;
@@ -1453,7 +1453,7 @@ int32_t redukt_backend_forward_batch_cdf_sym_wait(uint64_t ticket, uint32_t* out
     if (ok) memcpy(out_bounds, q->h_res, sizeof(uint32_t) * 3 * n_streams);
     q->ticket = 0;
     q->n = 0;
-    return ok ? BACKEND_OK : BACKEND_FORWARD_FAILED;
+    return ok ? (int32_t)BACKEND_OK : forward_failed();
 }
 
 int32_t redukt_backend_forward_batch_cdf_find(uint32_t n_streams, const uint32_t* slots, const uint32_t* tokens,

@@ -2697,6 +2697,11 @@ void StepRunner::clear() {
     plans_.clear();
 }
 
+void StepRunner::sync_parts() {
+    for (hipStream_t s : aux_)
+        if (s) (void)hipStreamSynchronize(s);
+}
+
 // The persistent kernel's arguments for (p, n), made on first use (at most 8 kept, the
 // least recently used evicted once the stream has finished with it).  out->shape.grid == 0
 // when the kernel cannot run on this device.

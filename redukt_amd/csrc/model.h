@@ -456,6 +456,9 @@ public:
     // event or device memory is created.
     hipError_t run_direct(const StepSource& src, Pool& p, const StepIO& io, hipStream_t st);
     void clear();
+    // Waits for the parts' own streams, which a step that failed between fork and join leaves
+    // running without st waiting for them.
+    void sync_parts();
     // Parts per step (1 .. kMaxParts) and the fewest streams a part may have; the streams
     // and events are created on first use.
     void set_split(uint32_t k, uint32_t min_part = kMinPartStreams) {
