@@ -101,6 +101,18 @@ float orc_lnf(float x) {
 
 /* tensor.rs:877-879: one lane of fast_exp_ps (a NaN lane is clamped to EXP_LO). */
 float orc_lane_expf(float x) { return orc_expf(isnan(x) ? -87.3365447505531f : x); }
+
+uint32_t orc_expf_differ(uint32_t first, uint32_t n, int lane, const float* got) {
+    uint32_t differ = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        const uint32_t b = first + i;
+        float x, want;
+        memcpy(&x, &b, 4);
+        want = lane ? orc_lane_expf(x) : orc_expf(x);
+        differ += memcmp(&want, &got[i], 4) != 0 && !(isnan(want) && isnan(got[i]));
+    }
+    return differ;
+}
 /* tensor.rs:883-885 */
 float orc_lane_sigmoidf(float x) { return 1.0f / (1.0f + orc_lane_expf(0.0f - x)); }
 #define lane_sigmoidf orc_lane_sigmoidf

@@ -40,6 +40,8 @@ enum {
 float orc_expf(float x);
 float orc_lnf(float x);
 float orc_lane_expf(float x);
+/* How many of got[0 .. n) are not expf (lane: lane_expf) of the float with bits first + i. */
+uint32_t orc_expf_differ(uint32_t first, uint32_t n, int lane, const float* got);
 float orc_sigmoidf(float x);
 float orc_softplus(float x);
 void  orc_softmax_into(const float* logits, float* out, int n);

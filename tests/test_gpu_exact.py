@@ -247,3 +247,54 @@ def test_streams_keep_their_bits_in_every_share(tmp_path, profile):
                 g = np.empty((n, dims.vocab), np.float32)
                 be.forward_batch(list(range(n)), [int(x) for x in toks[t, :n]], g)
                 assert np.array_equal(bits(g), bits(alone[t, :n])), (n, t)
+
+
+def rows_of_every_float(rng, norm_w, vocab):
+    """Head rows whose products and sums meet every kind of f32: magnitudes from the subnormals to
+    the largest, rows whose products are of one size (so that subnormal sums round and cancel),
+    zeros of both signs, and rows with infinities, NaN and overflows."""
+    d = norm_w.size
+    e = rng.integers(-149, 128, (vocab, 1)) + rng.integers(-3, 4, (vocab, d))
+    e = np.where(rng.random((vocab, 1)) < 0.5, e - np.round(np.log2(norm_w)), e)     # products of one size
+    w = np.ldexp(rng.choice([-1.0, 1.0], (vocab, d)) * rng.uniform(1.0, 2.0, (vocab, d)), e.astype(np.int64))
+    w = np.where(rng.random((vocab, d)) < 0.05, rng.choice([-0.0, 0.0], (vocab, d)), w)
+    odd = np.flatnonzero(rng.random(vocab) < 0.1)
+    w[odd, rng.integers(0, d, odd.size)] = rng.choice([np.inf, -np.inf, np.nan, 3.4028234e38, -3.4028234e38], odd.size)
+    with np.errstate(over="ignore"):
+        return w.astype(np.float32)
+
+
+@pytest.mark.parametrize("contract", [1, 2])
+def test_matrix_core_products_round_as_the_reference(tmp_path, contract):
+    """v_mfma_f32_4x4x1 is one fused multiply-add an output, rounded as fmaf rounds, and from an
+    accumulator of +0 the rounded product: 31 million products of operands of every kind
+    through an untied head, five streams and one, against the oracle's bits (a NaN for a NaN)."""
+    dims = rbin.MambaDims(vocab=8192, d_model=768, n_layer=1)
+    rng = np.random.default_rng(6)
+    flags = rbin.FLAG_UNTIED_HEAD
+    w = dict(synth.mamba_tensors(dims, 4, flags=flags))
+    head = [k for k, _ in rbin.tensor_order(dims, flags) if w[k].shape == (dims.vocab, dims.d_model) and k != "emb"]
+    w["norm_f_w"] = np.exp2(rng.integers(-40, 41, dims.d_model)).astype(np.float32)
+    w[head[0]] = rows_of_every_float(rng, w["norm_f_w"].astype(np.float64), dims.vocab)
+    path = str(tmp_path / "m.rbin")
+    rbin.write_rbin(path, dims, w.items(), flags=flags)
+    toks = [3, 1000, 8191, 0, 77]
+    orc = O.MambaOracle(path, O.ORC_PROFILE_FMA if contract == 2 else 0, cap=5)
+    want = np.ascontiguousarray(orc.forward(list(range(5)), toks), np.float32)
+    orc.close()
+    kinds = [np.isnan(want).mean(), np.isinf(want).mean(), ((np.abs(want) < 2.0 ** -126) & (want != 0)).mean()]
+    assert all(k > 0.005 for k in kinds) and np.isfinite(want).mean() > 0.7, kinds
+
+    def equal(g, c):
+        return (bits(g) == bits(c)) | (np.isnan(g) & np.isnan(c))
+
+    with ffi.PluginBackend(path, profile=EXACT | (FMA if contract == 2 else 0)) as be:
+        be.batch_init(5)
+        g = np.empty((5, dims.vocab), np.float32)
+        be.forward_batch(list(range(5)), toks, g)
+        assert equal(g, want).all(), np.argwhere(~equal(g, want))[:5]
+        be.batch_reset()
+        for s in range(5):
+            one = np.empty((1, dims.vocab), np.float32)
+            be.forward_batch([s], [toks[s]], one)
+            assert equal(one[0], want[s]).all(), s
