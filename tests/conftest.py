@@ -39,6 +39,18 @@ def oracle_plugin(tmp_path_factory):
     return so
 
 
+@pytest.fixture(scope="session")
+def fake_hip(tmp_path_factory):
+    """A stand-in for the HIP runtime (tests/fake_hip.c): loaded with RTLD_GLOBAL before
+    libredukt_gpu.so in a process of its own, it lets the library's host code run without a GPU."""
+    import subprocess
+
+    so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["gcc", "-O1", "-std=gnu11", "-shared", "-fPIC", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "fake_hip.c"), "-o", so, "-lpthread"], check=True)
+    return so
+
+
 # Worker pools stay within one GPU's share of host cores (16), whatever the machine
 # reports: the oracle's GEMV threads and the host library's coding threads.
 os.environ.setdefault("ORACLE_THREADS", str(min(os.cpu_count() or 1, 16)))

@@ -1,4 +1,4 @@
-/* A CPU stand-in for the HIP runtime, used by tests/test_failed_calls.py only.  Loaded with
+/* A CPU stand-in for the HIP runtime (the fake_hip fixture of tests/conftest.py).  Loaded with
  * RTLD_GLOBAL before libredukt_gpu.so, its definitions take the place of libamdhip64's for the
  * functions that library calls.  Device memory is host memory, kernels do nothing, and each
  * stream counts what was queued on it and how much of that is known to have ended: an event

@@ -9,6 +9,7 @@ group-64 profile on in_proj, out_proj and head 153,614,208; each stream reads an
 2 x (442,368 + 2,359,296) bytes of recurrent state per step, writes 201,120 bytes of logits
 and reads one 3,072-byte embedding row.
 """
+import json
 import os
 import subprocess
 import sys
@@ -48,3 +49,42 @@ def test_more_than_one_gpu_is_refused():
                        text=True, timeout=120)
     assert r.returncode == 2
     assert "one GPU" in r.stderr or "one process per GPU" in r.stderr
+
+
+PROBE_CHILD = r"""
+import ctypes, json, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+from redukt_amd import ffi
+used = {}
+with ffi.PluginBackend(sys.argv[2], profile=int(sys.argv[3])) as be:
+    be.batch_init(1)
+    out = np.empty((1, be.vocab), np.float32)
+    for name, cls in json.loads(sys.argv[4]).items():
+        be.probe_kernel(cls, (ctypes.c_void_p * 256)(*range(1, 257)))
+        be.forward_batch([0], [1], out)
+        used[name] = be.probe_used() // 2
+print(json.dumps(used))
+"""
+
+
+@pytest.mark.parametrize("arch,profile", [("mamba", p) for p in (0, 1, 6, 22, 64, 193)] +
+                         [("rwkv", p) for p in (0, 1, 2, 34, 64)])
+def test_launches_per_step_are_the_librarys(tmp_path, fake_hip, arch, profile):
+    # bench.py's probe pass records two events a launch and checks their number
+    from redukt_amd import ffi, rwkv, synth
+
+    path = str(tmp_path / "m.rbin")
+    if arch == "mamba":
+        dims = rbin.MambaDims(vocab=200, d_model=64, n_layer=3)
+        synth.write_synthetic_mamba(path, dims, seed=1)
+    else:
+        dims = rwkv.RwkvDims(vocab=200, d_model=128, n_layer=3)   # (more than one scale group a row)
+        rwkv.write_synthetic(path, dims, seed=1)
+    classes = ffi.KERNEL_CLASSES if arch == "mamba" else ffi.RWKV_KERNEL_CLASSES
+    classes = {k: v for k, v in classes.items() if k != "softmax"}
+    r = subprocess.run([sys.executable, "-c", PROBE_CHILD, fake_hip, path, str(profile), json.dumps(classes)], cwd=ROOT,
+                       capture_output=True, text=True, timeout=120, env={**os.environ, "PYTHONPATH": ROOT})
+    assert r.returncode == 0, r.stderr[-2000:]
+    used = json.loads(r.stdout.strip().splitlines()[-1])
+    assert used == {k: bench.launches_per_step(dims, k, arch == "mamba", profile) for k in classes}

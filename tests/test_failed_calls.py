@@ -71,14 +71,6 @@ print(json.dumps({"bad": bad, "seen": seen}))
 """
 
 
-@pytest.fixture(scope="module")
-def fake_hip(tmp_path_factory):
-    so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
-    subprocess.run(["gcc", "-O1", "-std=gnu11", "-shared", "-fPIC", "-I/opt/rocm/include",
-                    os.path.join(ROOT, "tests", "fake_hip.c"), "-o", so, "-lpthread"], check=True)
-    return so
-
-
 @pytest.mark.parametrize("arch,profile", [("mamba", 6), ("mamba", 64), ("rwkv", 2)])
 def test_a_failed_call_leaves_nothing_queued(tmp_path, fake_hip, arch, profile):
     from redukt_amd import rbin, rwkv, synth
