@@ -41,6 +41,7 @@ constexpr uint32_t kRbinMagic = 0x55504752u;  // "RGPU"
 constexpr uint32_t kFlagNormBias = 1u << 0;
 constexpr uint32_t kFlagUntiedHead = 1u << 1;
 constexpr int kMaxCols = 1024;  // d_model: activations of 32 streams staged in LDS, dt_rank in registers
+static_assert(kMaxCols <= kExactProductCols, "the reference-order tier's launches of several products");
 
 enum ModelKind : uint32_t { kKindNone = 0, kKindMamba = 1, kKindRwkv = 2 };
 
@@ -270,7 +271,7 @@ bool make_rowmat(RowMat& m, const float* w, int rows, int cols, int quant_group)
     std::vector<int8_t> q;
     std::vector<float> sc;
     m.group = quantize(w, rows, cols, quant_group, q, sc);
-    if (m.group % 32 != 0) return false;
+    if (m.group != kRowMatGroup && m.group != cols) return false;   // what k_gemv_e folds
     const int ng = cols / m.group;
     std::vector<int8_t> t(m.padded() * cols, 0);
     std::vector<float> ts(m.padded() * ng, 0.0f);
@@ -523,7 +524,7 @@ int load_rwkv(const std::string& path, uint32_t profile) {
     // A LoRA stage: tiled for the matrix cores, or laid out for the exact kernels of the
     // reference-order tier (whole 32-column blocks) or of the W8A8 tier.
     bool blocks32 = true;
-    for (uint32_t r : R.lora) blocks32 = blocks32 && r % 32 == 0 && r <= (uint32_t)kMaxCols;
+    for (uint32_t r : R.lora) blocks32 = blocks32 && r % 32 == 0;
     auto lora = [&](RLayer& L, int k, bool first, size_t rows, size_t cols) {
         std::vector<float> t = rd.read(rows * cols);
         if (G.r_exact && (first || blocks32))

@@ -488,7 +488,8 @@ template <int R, int C, int S, int EPI>
 const void* gemv_e_fn(const RowMat& w, bool fma) {
     if (w.group == 0) return fma ? (const void*)k_gemv_e<false, true, R, C, S, EPI, 0> : (const void*)k_gemv_e<false, false, R, C, S, EPI, 0>;
     if (w.group == w.cols) return fma ? (const void*)k_gemv_e<true, true, R, C, S, EPI, 0> : (const void*)k_gemv_e<true, false, R, C, S, EPI, 0>;
-    return fma ? (const void*)k_gemv_e<true, true, R, C, S, EPI, 2> : (const void*)k_gemv_e<true, false, R, C, S, EPI, 2>;
+    constexpr int kGB = kRowMatGroup / 32;   // (make_rowmat takes no other group)
+    return fma ? (const void*)k_gemv_e<true, true, R, C, S, EPI, kGB> : (const void*)k_gemv_e<true, false, R, C, S, EPI, kGB>;
 }
 
 // A wave's share of a product: 8 R rows and 4 C streams.
@@ -555,7 +556,8 @@ namespace {
 template <int AHEAD>
 const void* gemv_multi_fn(uint32_t n, Share s) {
     if (s.r == 1) return n == 1 ? (const void*)k_gemv_multi<1, 1, 1, AHEAD> : (const void*)k_gemv_multi<1, 1, 4, AHEAD>;
-    return (const void*)k_gemv_multi<2, 2, 4, AHEAD>;   // (rows of at most 1,024 columns: s.c = 2)
+    static_assert(32 * kExactProductCols <= (int)kELdsMax, "a share of 16 rows takes 8 streams (exact_share)");
+    return (const void*)k_gemv_multi<2, 2, 4, AHEAD>;
 }
 }  // namespace
 

@@ -53,6 +53,7 @@ struct GMat {
     size_t bytes() const;
 };
 
+constexpr int kRowMatGroup = 64;   // columns per scale of the reference's quantisation (or the whole row)
 // A [rows][cols] matrix for the reference-order tier: F32, or int8 with one f32 scale per
 // `group` columns (the values of the reference's own Q8wMatrix, src/domain/gemv.rs:244-273),
 // in the operand order of v_mfma_f32_4x4x1_16b_f32.  Rows are padded to whole 16-row tiles
@@ -64,7 +65,7 @@ struct GMat {
 // contiguous run.  Q8 scales: [t][cols / group][16 rows].
 struct RowMat {
     int rows = 0, cols = 0;
-    int group = 0;        // 0: F32; Q8: columns per scale
+    int group = 0;        // 0: F32; Q8: columns per scale, kRowMatGroup or the whole row
     void* w = nullptr;
     float* scales = nullptr;
     __host__ __device__ int tiles() const { return (rows + kRowTile - 1) / kRowTile; }
@@ -245,7 +246,7 @@ struct RLayer {
     TMat l2[4];                       // second LoRA stages [d][rank] (F32): w2, a2, g2, v2
     TMat fk, fv;                      // [d_ffn][d], [d][d_ffn]
     // The LoRA stages of the W8A8 tier; of the reference-order tier in e_x1 and e_x2 (x2
-    // instead where a rank is not a multiple of 32, or above 1,024).  l1 and l2 stay empty there.
+    // instead where a rank is not a multiple of 32).  l1 and l2 stay empty there.
     LMat x1[4], x2[4];
     RowMat e_x1[4], e_x2[4];
     RowMat e_r, e_k, e_v, e_o, e_fk, e_fv;   // the reference-order tier's projections (the TMats stay empty there)
@@ -395,10 +396,11 @@ struct ExactStep final : StepSource {
 enum ExactEpi : int { EXACT_STORE = 0, EXACT_RESID = 2, EXACT_RELU2 = 3 };
 Launch exact_gemv_launch(const RowMat& w, const float* act, uint32_t n, float* out, uint32_t ostride, int epi,
                          uint32_t cls);
-// Up to kExactProducts such products of at most 1,024 columns, none reading another's output,
+// Up to kExactProducts such products of at most kExactProductCols columns, none reading another's output,
 // in one launch: product k's input rows are x + b * ldx, its outputs take the activation act
 // (rwkv_common.h).
 constexpr int kExactProducts = 7;
+constexpr int kExactProductCols = 1024;   // the loader's limit of d_model; a LoRA rank is 512 at most
 struct ExactProduct {
     const RowMat* w;
     const float* x;
