@@ -601,9 +601,16 @@ void dev_free_all() {
 constexpr size_t kOutChunkTarget = (size_t)4 << 20;
 // Logits of up to this many bytes are written by the head straight into pinned host memory: no
 // DMA behind the step (8 us each, in two chunks) and no copy threads, but the head's own stores
-// cross the bus, at about 17 GB/s.  us a call, with the DMAs / direct (Mamba-130M int8 through
-// the C ABI): 1 stream 420 / 376, 2 427 / 391, 4 430 / 411, 8 449 / 470, 32 578 / 854; RWKV-7
-// int8 1 stream 547 / 507, 4 (1 MB) 569 / 574; the reference-order tier 1 stream 738 / 698.
+// cross the bus, at about 17 GB/s.  us a call through the C ABI, with the DMAs / direct
+// (Mamba-130M, 50,280 symbols, at 1 and 4 streams, 786 KB; RWKV-7 0.1B, 65,536, at 1 and 3,
+// 768 KB), each head of the tiers: Mamba int8 per row 415 / 371 and 422 / 401, groups of 64
+// 449 / 405 and 453 / 433, F32 629 / 583 and 634 / 607, wavefront GEMV int8 404 / 360 and 527 /
+// 488, F32 542 / 494 and 676 / 633, reference order F32 856 / 811 and 890 / 853, int8 747 / 704 and
+// 769 / 744; RWKV-7 int8 542 / 503 and 561 / 541, F32 722 / 676 and 739 / 705, W8A8 778 / 735 and
+// 794 / 765, reference order 785 / 738 and 810 / 767.  Many streams of a small vocabulary: 256
+// symbols, 64 / 256 / 800 streams, int8 530 / 485, 941 / 900, 2,011 / 1,977; 4,096 symbols, 54
+// streams 553 / 524.  Above it the DMAs win: int8 8 streams (1.6 MB) 449 / 470, 32 578 / 854,
+// RWKV-7 4 streams (1 MB) 569 / 574.
 constexpr size_t kDirectOutBytes = (size_t)900 << 10;
 constexpr size_t kOutMaxChunks = 4;
 constexpr size_t kOutRoundBytes = (size_t)32 << 20;
@@ -623,7 +630,7 @@ bool out_stage_alloc(Pool& p, size_t out_bytes) {
     return true;
 }
 
-// The host side of the queued calls' buffers (the device inputs are carved with the pool).
+// The queued calls' inputs and results, which the device reads and writes in place, and events.
 bool queued_alloc(Pool& p, size_t n) {
     for (Pool::Queued& q : p.queued) {
         if (hipHostMalloc((void**)&q.h_in, sizeof(uint32_t) * 3 * n, hipHostMallocDefault) != hipSuccess) {

@@ -265,12 +265,14 @@ __global__ __launch_bounds__(kCdfBlock) void k_cdf_exp(CdfArgs a) {
 // by term.  The running sum of these rows is NaN or stays below 2^24 (each term <= 1, n < 2^24),
 // so the grid is always finer than 1.
 //
-// Bound by latency.  128 rows of 50,280 normal logits of standard deviations 1 to 4: 57 us (67
-// with the shares after the sums), where 4,096 terms of the whole workgroup a round in order
-// (two barriers, 1.7 us each, about 46 rounds a row) took 121; the whole CDF 175 -> 112.  Of a
-// row, each sum: 1.8 us to classify, 7 to count (51 MB of e over all rows at 7 TB/s; the second
-// sum 8 to 17, by how many of its terms are ties), 10 to 14 in the chain, whose lone wave issues
-// at a third of the vector rate: about 1.3 us for each uncounted segment with the run before it.
+// Bound by latency.  128 rows of 50,280 normal logits of standard deviations 1 to 4: 65 us, about
+// 7 of them the shares after the sums, where 4,096 terms of the whole workgroup a round in order
+// (two barriers, 1.7 us each, about 46 rounds a row) took 120 without the shares; the whole call
+// 171 -> 102 us.  Of a row, each sum: 1.8 us to classify, 7 to count (51 MB of e over all rows at
+// 7 TB/s; the second sum 8 to 17, by how many of its terms are ties), 10 to 14 in the chain, whose
+// lone wave issues at a third of the vector rate: about 1.3 us for each uncounted segment with
+// the run before it.
+
 // The same value in every lane, made visibly uniform (scalar registers): the round loop's
 // control values come from LDS, and without this the compiler treats the loop as divergent
 // (exec masking, and copies of the prefetched terms that wait for their loads every round).
@@ -743,7 +745,7 @@ __device__ void freq_part(const uint32_t* __restrict__ p, uint32_t n, uint32_t c
 
 // A row of one segment (a byte vocabulary): one wave adds its terms in order, both times from
 // the same registers, and takes their shares from there.  Bound by the two chains of adds and the
-// launches: the whole CDF of 128 / 512 rows of 256 takes 13.7 / 14.4 us, 19.5 for 128 rows through
+// launches: the whole call for 128 / 512 rows of 256 takes 13.5 / 14.4 us, 19.6 / 28.5 through
 // k_cdf_sums; two segments gain from it no more (its second one would be another chain of 256).
 __global__ __launch_bounds__(64) void k_cdf_sums_short(CdfArgs a) {
     __shared__ double terms[kSegTerms];
@@ -821,8 +823,6 @@ struct RowFix {
     uint64_t most;     // that element's frequency before it
     uint32_t total;    // cdf[n]
 };
-// Chunk c's first cumulative frequency (u32, wrapping, as the host's sum; each frequency is 1
-// and its share).
 __device__ __forceinline__ RowFix row_fix(const CdfArgs& a, uint32_t row) {
     RowFix x;
     x.f = freq_row(a.sums[row], a.n);
@@ -838,6 +838,8 @@ __device__ __forceinline__ RowFix row_fix(const CdfArgs& a, uint32_t row) {
     x.total = (uint32_t)((int64_t)(a.n + used) + x.diff);
     return x;
 }
+// Chunk c's first cumulative frequency (u32, wrapping, as the host's sum; each frequency is 1
+// and its share).
 __device__ __forceinline__ uint32_t chunk_offset(const CdfArgs& a, uint32_t row, uint32_t c, const RowFix& x) {
     const ChunkPart* pr = a.part + (size_t)row * a.chunks;
     uint32_t offset = 0;

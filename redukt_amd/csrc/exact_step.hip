@@ -191,8 +191,8 @@ __device__ __forceinline__ float madd(float w, float x, float acc) {
 // (of four streams) times w[h][j] (of the lane's row h) added to acc[h][q] in the contract's
 // arithmetic.  v_mfma_f32_4x4x1_16b_f32 is sixteen blocks of a 4 x 1 times 1 x 4 product: each
 // of its 256 outputs is one fused multiply-add, rounded once as fmaf rounds (subnormals,
-// infinities and zeros too: checked bit for bit on 21 million random operands).  That is
-// contract 2; contract 1 takes the rounded products from it (accumulator +0; an exact product
+// infinities and zeros too: tests/test_gpu_exact.py holds 31 million products of operands of
+// every kind to the oracle's bits).  That is contract 2; contract 1 takes the rounded products from it (accumulator +0; an exact product
 // of -0 comes out +0, which an accumulator that starts at +0 and so never holds -0 cannot
 // tell apart) and adds them on the vector unit, eight products issued before the first add.
 // S of the four streams are live.
@@ -305,8 +305,8 @@ constexpr int kEAheadShort = 4;   // the same where no row of a launch of severa
 // the whole row is one sum).
 //
 // Bound by vector instructions once the batch fills the chip (the head of 100 F32 streams,
-// contract 1: 91 % of the cycles issue one; two thirds of them are the adds themselves), by
-// the chain of dependent products and the load latencies below that.  The version before this
+// contract 1: they take 86 % of the cycles that its CUs are busy, SQ_ACTIVE_INST_VALU over
+// SQ_BUSY_CU_CYCLES; 71 % of them are the adds themselves), by the chain of dependent products and the load latencies below that.  The version before this
 // one (eight lanes an output on the vector unit, each product reading its activation from
 // LDS) was bound by LDS.  us a launch, before and now: F32 contract 1 at 100 streams in_proj
 // 28.5 -> 19.6, x_proj 16.6 -> 6.9, out_proj 19.6 -> 12.0, head 357 -> 187; int8 groups of 64

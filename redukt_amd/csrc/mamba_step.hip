@@ -717,7 +717,7 @@ __device__ __forceinline__ void apply_row_scales(const TMat& w, int t, f32x4 (&a
 struct EmbedArgs {
     TMat emb;
     float* x;                  // [n][d]
-    const uint32_t* tokens;    // caller's device pointers, at this part's first row
+    const uint32_t* tokens;    // the caller's device pointers or pinned memory, at this part's first row
     const uint32_t* slots_in;
     uint32_t* slots;           // validated copy used by the rest of the step
     uint32_t n, cap;

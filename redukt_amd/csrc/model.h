@@ -289,7 +289,8 @@ struct ModelView {
     bool exact_scan;        // scan decay factors by the portable exp (else the hardware exp2)
 };
 
-// One step's inputs.  slots/tokens/out are device pointers; `check` validates slots
+// One step's inputs.  slots/tokens/out are memory that the device reads and writes: the
+// caller's device pointers or the pool's pinned host memory; `check` validates slots
 // and tokens on the device into *err (bit 0: out of range, bit 1: duplicate slot).
 // A step may run as several parts (sub-batches of whole 16-stream groups): a part covers
 // batch rows [b0, b0 + n) of the step's n_all rows; slots, tokens and out always point at

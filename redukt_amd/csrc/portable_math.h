@@ -43,7 +43,7 @@ RDK_HD float round_even(float x) {
 // (tensor.rs:765-794).
 #if defined(__HIP_DEVICE_COMPILE__)
 // On the device in 24 vector instructions instead of 37, with the same bits for every one of the
-// 2^32 inputs (compared): a NaN takes the lower bound (the lane rule below), the rounding is one
+// 2^32 inputs (tests/test_gpu_math.py compares them all): a NaN takes the lower bound (the lane rule below), the rounding is one
 // v_rndne (it may give -0 for +0, which leaves the result), and the scale one v_ldexp (one
 // rounding, as the multiplication by 2^n).  The reference-order scan, 18 of them a thread: 32
 // streams 6.9 -> 5.6 us, 100 streams 10.8 -> 10.0 (with its dt_rank fixed); the softmax of 128
