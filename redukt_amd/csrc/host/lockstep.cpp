@@ -584,8 +584,8 @@ extern "C" int32_t redukt_lockstep_open(const char* plugin_path, const char* wei
     ls->uniform.assign(size_t(ls->vocab) + 1, 0u);
     redukt_cdf_uniform(ls->vocab, ls->uniform.data());
     // The device CDF is the faster path wherever the plugin has it (Mamba-130M int8, 16 host
-    // threads: forward_batch_cdf 0.93 ms per step at 32 streams against 0.58 ms forward +
-    // 0.71 ms host CDF, 1.77 ms at 128 streams against 1.27 + 2.60 ms).
+    // threads, a step with its coding: whole device rows 0.71 ms at 32 streams against 1.5 with
+    // host CDFs, 1.41 ms at 128 against 3.87).
     ls->device_cdf = ls->api.forward_batch_cdf != nullptr && slots >= kDeviceCdfFrom;
     // REDUKT_LOCKSTEP_CDF_SYM=0: compression and decompression take whole device CDF rows.
     const char* e = getenv("REDUKT_LOCKSTEP_CDF_SYM");

@@ -1421,7 +1421,8 @@ const void* scan_fn(bool q8dt, bool fast, int dr, int nxb, uint32_t spt) {
 }
 
 // The reference-order tier's, specialised for Mamba-130M's dt_rank in the same way: 48 fixed
-// terms of the dt_proj dot instead of 64 with a test each.
+// terms of the dt_proj dot instead of 64 with a test each (32 int8 streams 6.7 -> 5.5 us a launch,
+// 100 F32 streams 10.9 -> 10.0).
 template <bool Q8DT, bool FMA>
 const void* scan_exact_fn(bool m130) {
     return m130 ? (const void*)k_scan<Q8DT, false, 48, 1, 1, FMA> : (const void*)k_scan<Q8DT, false, 0, 1, 1, FMA>;

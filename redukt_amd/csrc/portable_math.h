@@ -46,8 +46,8 @@ RDK_HD float round_even(float x) {
 // 2^32 inputs (tests/test_gpu_math.py compares them all): a NaN takes the lower bound (the lane rule below), the rounding is one
 // v_rndne (it may give -0 for +0, which leaves the result), and the scale one v_ldexp (one
 // rounding, as the multiplication by 2^n).  The reference-order scan, 18 of them a thread: 32
-// streams 6.9 -> 5.6 us, 100 streams 10.8 -> 10.0 (with its dt_rank fixed); the softmax of 128
-// rows of 50,280 22.5 -> 20.8.
+// streams 6.3 -> 5.5 us, 100 streams 10.6 -> 10.0; the softmax of two parts of 64 rows of 50,280,
+// a part 22.0 -> 20.8.
 RDK_HD float exp_clamped_f(float x) {
     x = x > -87.3365447505531f ? x : -87.3365447505531f;
     x = __builtin_amdgcn_fmed3f(x, -87.3365447505531f, 88.3762626647949f);
