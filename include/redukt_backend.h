@@ -184,8 +184,8 @@ int32_t redukt_backend_forward_batch_cdf_find(uint32_t n_streams, const uint32_t
 
 /* forward_batch_cdf_sym in two halves, so that a caller that knows its next inputs
  * (compression) can queue the next step before it has used this one's results: _submit
- * validates and queues the step, the device CDF and the copy of the three values per
- * stream, and returns at once with *ticket naming the call; _wait(ticket) waits for that
+ * validates and queues the step, the device CDF and the kernel that writes the three values
+ * per stream into host memory, and returns at once with *ticket naming the call; _wait(ticket) waits for that
  * call and writes out_bounds (3 u32 a stream, n_streams as submitted).  At most two calls
  * are in flight: a third _submit before one of them is waited for is refused.  Calls run in
  * submission order, after and before every other entry point's work, and each sees the

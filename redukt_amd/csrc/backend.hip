@@ -964,8 +964,8 @@ bool copy_out(Pool& p, void* dst, const void* src, size_t bytes) {
 
 // pool_forward semantics (mamba_cuda.cu:604-635): validate on the host (nothing is
 // launched on INVALID_ARGUMENT), put slots and tokens into pinned memory, enqueue the step,
-// which reads them there, copy the n rows back to the caller (through pinned staging,
-// chunked) and wait.
+// which reads them there, wait, and copy the n rows to the caller: out of pinned memory where the
+// head wrote them there (kDirectOutBytes), else through pinned staging, chunked (copy_out).
 int pool_forward(Pool& p, uint32_t n, const uint32_t* slots, const uint32_t* tokens, float* out, bool probs) {
     memset(p.seen, 0, p.cap);
     for (uint32_t b = 0; b < n; b++) {
